@@ -41,6 +41,7 @@ namespace hif8 {
 namespace {
 
 constexpr int kBK = 64;  // bytes (= bf16 elements) of K per stage
+constexpr int64_t kMaxSkinnyK = 0x7FFFFF00ll;  // k rounded up to 64 fits int
 constexpr int kMaxDmaK = 1 << 23;  // gemm_dma_kernel: a tile's rows in 32-bit byte offsets
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -1003,17 +1004,41 @@ int launch_plan(const LinearArgs &a, const GemmPlan &p, const void *act, int spl
 
 }  // namespace
 
+namespace {
+
+// Whether a call runs gemm_skinny_kernel: every K that the tiles do not take,
+// up to 64 rows (one row tile reads the weight once), and more rows while the
+// 64 x 32 blocks still fit the CUs in one round and K is short.  MI355X, whole
+// call against the 128 x 128 tiles: M = 64 24576 x 4096 44.6 vs 54.5 us, 4096
+// x 4096 15.4 vs 25.3; M = 128 4096 x 4096 18.5 vs 28.6; M = 256 2048 x 4096
+// 18.1 vs 27.9; but M = 128 4096 x 12288 43 vs 37.7 and 24576 x 4096 70 vs 59.
+bool skinny_rule(int64_t m, int64_t n, int64_t k) {
+  if (k > kMaxSkinnyK) return false;
+  return k % kBK != 0 || m <= 64 || (k <= 8192 && (n + 31) / 32 * ((m + 63) / 64) <= 256);
+}
+
+}  // namespace
+
 size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m <= 4 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > 0x7FFFFFFFll || n <= 0 || k <= 0 || k % kBK)
     return 0;
+  if (skinny_rule(m, n, k)) return skinny_workspace_size(m, k);
   const GemmPlan p = plan_gemm(m, n, k);
   return p.a_bytes + p.w_bytes + p.part_bytes;
+}
+
+size_t gemm_scratch_size(int64_t m, int64_t n, int64_t k) {
+  if (m <= 4 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > 0x7FFFFFFFll || n <= 0 || k <= 0) return 0;
+  return k % kBK ? (skinny_rule(m, n, k) ? skinny_workspace_size(m, k) : 0) : gemm_workspace_size(m, n, k);
 }
 
 int launch_gemm(const LinearArgs &a) {
   if (a.act_kind != kActCodes)
     return fail(HIF8_ERR_UNSUPPORTED, "soft_hif8 GEMM takes uint8 activation codes");
   const bool tiled = a.k % kBK == 0 && aligned(a.act, 16) && aligned(a.weight, 16);
+  if (skinny_rule(a.m, a.n, a.k) && a.workspace && a.workspace_bytes >= skinny_workspace_size(a.m, a.k) &&
+      aligned(a.workspace, 256))
+    return launch_gemm_skinny(a);
   if (!tiled) {
     const dim3 grid(unsigned((a.n + 255) / 256), unsigned(a.m));
     gemm_simple_kernel<<<grid, 256, 0, a.stream>>>(

@@ -120,6 +120,10 @@ extern "C" size_t soft_hif8_gemm_workspace_size(int64_t m, int64_t n, int64_t k)
   return gemm_workspace_size(m, n, k);
 }
 
+extern "C" size_t soft_hif8_gemm_scratch_size(int64_t m, int64_t n, int64_t k) {
+  return gemm_scratch_size(m, n, k);
+}
+
 extern "C" int soft_hif8_gemm_with_workspace(const uint8_t *activation, const uint8_t *weight,
                                              const float *token_scale, const float *channel_scale,
                                              const void *bias, int bias_dtype, void *out,

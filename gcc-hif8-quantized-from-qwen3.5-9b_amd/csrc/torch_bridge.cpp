@@ -198,9 +198,9 @@ at::Tensor SoftHif8Gemm(const at::Tensor &activation, const at::Tensor &weight, 
   const c10::OptionalDeviceGuard guard(activation.device());
   const int64_t m = activation.size(0), n = weight.size(0), k = activation.size(1);
   auto out = at::empty({m, n}, activation.options().dtype(output_dtype));
-  // Split-K workspace from the stream-ordered caching allocator, as the
+  // Workspace (bf16 activation, split-K partials) from the stream-ordered caching allocator, as the
   // reference takes its ACLNN workspace (hif8_native.cpp:202-226).
-  const size_t ws_bytes = soft_hif8_gemm_workspace_size(m, n, k);
+  const size_t ws_bytes = soft_hif8_gemm_scratch_size(m, n, k);
   at::Tensor ws;
   if (ws_bytes) ws = at::empty({int64_t(ws_bytes)}, activation.options().dtype(at::ScalarType::Byte));
   const void *bias_ptr = bias.has_value() ? bias->data_ptr() : nullptr;

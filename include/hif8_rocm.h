@@ -147,6 +147,14 @@ int soft_hif8_gemm(const uint8_t *activation, const uint8_t *weight, const float
 size_t soft_hif8_gemm_workspace_size(int64_t m, int64_t n, int64_t k);
 
 /*
+ * The workspace with which soft_hif8_gemm_with_workspace runs fastest: the size
+ * above, and for K that is no multiple of 64, where that is 0 and a call without
+ * workspace computes one output per thread, the bf16 activation fragments with
+ * which the call runs on the matrix cores.
+ */
+size_t soft_hif8_gemm_scratch_size(int64_t m, int64_t n, int64_t k);
+
+/*
  * soft_hif8_gemm with a caller-owned workspace: the second phase,
  * aclnnSoftHif8Gemm(workspace, size, executor, stream) (hif8_native.cpp:228-239,386-425).
  * With workspace_bytes >= soft_hif8_gemm_workspace_size(m, n, k) (256-byte aligned)

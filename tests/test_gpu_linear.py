@@ -113,6 +113,29 @@ def test_gemm_shapes_and_tails(native_ops, device, rows, channels, k):
         _check(y, want - bias + rounded)
 
 
+@pytest.mark.parametrize("rows,channels,k", [
+    # K: below, at and past a 64-code step, a partial step alone in its round of
+    # wavefronts, odd rows; M and N: edges of the 16-row tiles and of a 64-row tile.
+    (5, 1, 64), (16, 15, 63), (17, 33, 65), (64, 16, 1024), (65, 40, 130), (48, 100, 1089), (130, 18, 100),
+    (20, 4200, 192), (70, 2100, 333), (256, 64, 448),
+])
+def test_few_row_and_ragged_gemm(native_ops, device, rows, channels, k):
+    """The streaming GEMM (up to 64 rows, or any K): values against the float64
+    oracle, and NaN / Inf weight codes only in the outputs whose rows hold them
+    (a partial step reads next to the following row)."""
+    a = random_codes((rows, k), seed=rows + k)
+    w = random_codes((channels, k), seed=channels + k)
+    w[channels // 2] = 0x80  # a row of NaN codes after and before finite ones
+    ts = np.full(rows, 1e-3, np.float32)
+    cs = np.linspace(1e-3, 2e-3, channels, dtype=np.float32)
+    keep = np.arange(channels) != channels // 2
+    want = o.linear_u8_u8(a, ts, w[keep], cs[keep], None) if keep.any() else np.zeros((rows, 0))
+    y = native_ops.soft_hif8_gemm(_t(a, device), _t(w, device), _t(ts, device), _t(cs, device), None, torch.bfloat16)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(y[:, channels // 2]).all())
+    _check(y[:, torch.from_numpy(keep).to(device)], want)
+
+
 @pytest.mark.parametrize("m", [1, 4])
 @pytest.mark.parametrize("n,k", LAYER_SHAPES)
 def test_decode_gemv_config_shapes(native_ops, device, m, n, k):
