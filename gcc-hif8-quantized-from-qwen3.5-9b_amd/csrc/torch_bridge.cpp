@@ -876,6 +876,55 @@ at::Tensor Hif8GdnDecodeHead(const at::Tensor &conv, const at::Tensor &mixed, co
   return out;
 }
 
+// The gated delta rule over many tokens: q, k [B, H, T, dk], v [B, H, T, dv], g,
+// beta [B, H, T] of any strides (copied where rows are not contiguous or q / k
+// rows not 16-byte aligned), state [B, H, dk, dv] contiguous, updated in place.
+at::Tensor Hif8GatedDelta(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v, const at::Tensor &g,
+                          const at::Tensor &beta, at::Tensor &state) {
+  for (auto *t : {&q, &k, &v, &g, &beta}) {
+    TORCH_CHECK(t->is_cuda() && t->device() == state.device(), "hif8_gated_delta: tensors must be on one device");
+    TORCH_CHECK(t->scalar_type() == at::kFloat, "hif8_gated_delta: float32 tensors expected");
+  }
+  CheckContiguousDevice(state, "state");
+  TORCH_CHECK(state.scalar_type() == at::kFloat && state.dim() == 4 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
+                  g.dim() == 3 && beta.dim() == 3,
+              "hif8_gated_delta: operand ranks");
+  const int64_t batch = v.size(0), heads = v.size(1), tokens = v.size(2), dv = v.size(3), dk = k.size(3);
+  const at::IntArrayRef rows[] = {k.sizes(), q.sizes()};
+  for (const auto &r : rows)
+    TORCH_CHECK(r[0] == batch && r[1] == heads && r[2] == tokens && r[3] == dk, "hif8_gated_delta: q / k shape");
+  TORCH_CHECK(g.sizes() == v.sizes().slice(0, 3) && beta.sizes() == g.sizes(), "hif8_gated_delta: g / beta shape");
+  TORCH_CHECK(state.size(0) == batch && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv,
+              "hif8_gated_delta: state shape");
+  const c10::OptionalDeviceGuard guard(state.device());
+  auto rowwise = [](const at::Tensor &t, bool vec) {
+    bool ok = t.stride(3) == 1;
+    if (vec) {
+      ok = ok && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+      for (int i = 0; i < 3; ++i) ok = ok && t.stride(i) % 4 == 0;
+    }
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+  };
+  const at::Tensor qc = rowwise(q, true), kc = rowwise(k, true), vc = rowwise(v, false);
+  auto out = at::empty({batch, heads, tokens, dv}, v.options());
+  const size_t ws_bytes = hif8_gated_delta_workspace_size(batch, heads, tokens, dk, dv);
+  auto ws = at::empty({int64_t(ws_bytes)}, v.options().dtype(at::ScalarType::Byte));
+  int64_t strides[18];
+  const at::Tensor *order[] = {&qc, &kc, &vc, &g, &beta, &out};
+  for (int i = 0; i < 6; ++i)
+    for (int j = 0; j < 3; ++j) strides[3 * i + j] = order[i]->stride(j);
+  CheckStatus(hif8_gated_delta(qc.data_ptr<float>(), kc.data_ptr<float>(), vc.data_ptr<float>(), g.data_ptr<float>(),
+                               beta.data_ptr<float>(), strides, state.data_ptr<float>(), out.data_ptr<float>(), batch,
+                               heads, heads, tokens, dk, dv, ws.data_ptr(), ws_bytes, CurrentStream(state.device())),
+              "hif8_gated_delta");
+  return out;
+}
+
+at::Tensor Hif8GatedDeltaMeta(const at::Tensor &, const at::Tensor &, const at::Tensor &v, const at::Tensor &,
+                              const at::Tensor &, at::Tensor &) {
+  return at::empty(v.sizes(), v.options());
+}
+
 // hif8_gdn_decode_step with the b/a projection of x folded in; shapes the
 // fused kernel does not take run hif8_bf16_gemv + hif8_gdn_decode_step.
 at::Tensor Hif8GdnDecodeToken(const at::Tensor &mixed, const at::Tensor &x, const at::Tensor &ba_weight,
@@ -1110,6 +1159,7 @@ TORCH_LIBRARY(vllm_ascend_hif8, m) {
   m.def("hif8_gate_up_silu_mul_quant(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor input_scale) -> (Tensor, Tensor)");
   m.def("hif8_gdn_decode_token(Tensor mixed_qkvz, Tensor x, Tensor ba_weight, Tensor conv_weight, Tensor(a!) conv_state, Tensor a_log, Tensor dt_bias, Tensor(b!) rec_state, Tensor out_norm, int k_heads, int v_heads, int k_dim, int v_dim, float eps) -> Tensor");
   m.def("hif8_linear_conv(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor conv_weight, Tensor(a!) conv_state) -> (Tensor, Tensor)");
+  m.def("hif8_gated_delta(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state) -> Tensor");
   m.def("hif8_gdn_decode_head(Tensor conv, Tensor mixed_qkvz, Tensor x, Tensor ba_weight, Tensor a_log, Tensor dt_bias, Tensor(a!) rec_state, Tensor out_norm, int k_heads, int v_heads, int k_dim, int v_dim, float eps) -> Tensor");
 }
 
@@ -1135,6 +1185,7 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, CUDA, m) {
   m.impl("hif8_gdn_decode_token", &Hif8GdnDecodeToken);
   m.impl("hif8_gate_up_silu_mul_quant", &Hif8GateUpSiluMulQuant);
   m.impl("hif8_linear_conv", &Hif8LinearConv);
+  m.impl("hif8_gated_delta", &Hif8GatedDelta);
   m.impl("hif8_gdn_decode_head", &Hif8GdnDecodeHead);
   m.impl("soft_hif8_gemm_decoded_weight", &SoftHif8GemmDecodedWeight);
   m.impl("hif8_decode_bf16", &Hif8DecodeBf16);
@@ -1164,6 +1215,7 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, Meta, m) {
   m.impl("hif8_gdn_decode_token", &Hif8GdnDecodeTokenMeta);
   m.impl("hif8_gate_up_silu_mul_quant", &Hif8GateUpSiluMulQuantMeta);
   m.impl("hif8_linear_conv", &Hif8LinearConvMeta);
+  m.impl("hif8_gated_delta", &Hif8GatedDeltaMeta);
   m.impl("hif8_gdn_decode_head", &Hif8GdnDecodeHeadMeta);
 }
 

@@ -476,6 +476,25 @@ int hif8_gdn_decode_token(const uint16_t *mixed_qkvz, int64_t ld, const uint16_t
                           int64_t batch, int64_t k_heads, int64_t v_heads, int64_t k_dim, int64_t v_dim,
                           int64_t conv_width, float eps, hif8_stream_t stream);
 
+/*
+ * The gated delta rule of a linear-attention layer over `tokens` tokens (FP32):
+ *   S <- e^g S;  S <- S + k (beta (v - S^T k))^T;  o = S^T q
+ * per request and value head, computed in chunks of 64 tokens.  q and k are
+ * normalised and scaled by the caller; value head h reads key head
+ * h / (heads / k_heads).
+ *   strides  18 element strides: (batch, head, token) of q, k, v, g, beta and out;
+ *            the last dimension of q, k, v and out is contiguous, q and k rows are
+ *            16-byte aligned (strides % 4 == 0)
+ *   state    [batch, heads, k_dim, v_dim] contiguous, updated in place
+ * k_dim 64 or 128, v_dim % 16 == 0 and <= 256; workspace of
+ * hif8_gated_delta_workspace_size bytes, 256-byte aligned.
+ */
+size_t hif8_gated_delta_workspace_size(int64_t batch, int64_t heads, int64_t tokens, int64_t k_dim, int64_t v_dim);
+int hif8_gated_delta(const float *q, const float *k, const float *v, const float *g, const float *beta,
+                     const int64_t *strides, float *state, float *out, int64_t batch, int64_t heads, int64_t k_heads,
+                     int64_t tokens, int64_t k_dim, int64_t v_dim, void *workspace, size_t workspace_bytes,
+                     hif8_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
