@@ -35,7 +35,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "linear.h"
+#include "gemm_operand.h"
 
 namespace hif8 {
 namespace {
@@ -1006,6 +1006,17 @@ int launch_plan(const LinearArgs &a, const GemmPlan &p, const void *act, int spl
 
 namespace {
 
+// The GEMM of a plan whose workspace holds the bf16 activation, with w_pre the
+// bf16 weight after it, and room for the split partials last.
+int launch_prepared(const LinearArgs &a, const GemmPlan &p, uint8_t *ws) {
+  const uint16_t *abf = reinterpret_cast<const uint16_t *>(ws);
+  float *partial = p.part_bytes ? reinterpret_cast<float *>(ws + p.a_bytes + p.w_bytes) : nullptr;
+  const int splits = p.part_bytes ? p.splits : 1;
+  if (p.w_pre)
+    return launch_bf16_operands(a, p, abf, reinterpret_cast<const uint16_t *>(ws + p.a_bytes), splits, partial);
+  return launch_plan<true>(a, p, abf, splits, partial);
+}
+
 // Whether a call runs gemm_skinny_kernel: every K that the tiles do not take,
 // up to 64 rows (one row tile reads the weight once), and more rows while the
 // 64 x 32 blocks still fit the CUs in one round and K is short.  MI355X, whole
@@ -1037,8 +1048,11 @@ int launch_gemm(const LinearArgs &a) {
     return fail(HIF8_ERR_UNSUPPORTED, "soft_hif8 GEMM takes uint8 activation codes");
   const bool tiled = a.k % kBK == 0 && aligned(a.act, 16) && aligned(a.weight, 16);
   if (skinny_rule(a.m, a.n, a.k) && a.workspace && a.workspace_bytes >= skinny_workspace_size(a.m, a.k) &&
-      aligned(a.workspace, 256))
-    return launch_gemm_skinny(a);
+      aligned(a.workspace, 256)) {
+    uint16_t *act = static_cast<uint16_t *>(a.workspace);
+    const int st = launch_decode_fragments(a, act);
+    return st ? st : launch_gemm_skinny(a, act);
+  }
   if (!tiled) {
     const dim3 grid(unsigned((a.n + 255) / 256), unsigned(a.m));
     gemm_simple_kernel<<<grid, 256, 0, a.stream>>>(
@@ -1061,13 +1075,35 @@ int launch_gemm(const LinearArgs &a) {
                                                    wchunks);
   const int st = check_launch(p.w_pre ? "soft_hif8 GEMM (activation and weight decode)"
                                       : "soft_hif8 GEMM (activation decode)");
+  return st ? st : launch_prepared(a, p, ws);
+}
+
+size_t gemm_static_workspace_size(int64_t m, int64_t n, int64_t k) {
+  if (m <= 4 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > kMaxSkinnyK || n <= 0 || k <= 0) return 0;
+  const size_t scales = (size_t(m) * sizeof(float) + 255) / 256 * 256;
+  // Fragments also where a weight that is not 16-byte aligned keeps the tiles away.
+  return scales + std::max(skinny_workspace_size(m, k), k % kBK ? 0 : gemm_workspace_size(m, n, k));
+}
+
+int launch_gemm_static(const LinearArgs &a) {
+  float *row_scale = static_cast<float *>(a.workspace);
+  uint8_t *ws = static_cast<uint8_t *>(a.workspace) + (size_t(a.m) * sizeof(float) + 255) / 256 * 256;
+  uint16_t *act = reinterpret_cast<uint16_t *>(ws);
+  const bool fragments = skinny_rule(a.m, a.n, a.k) || !aligned(a.act, 16) || !aligned(a.weight, 16);
+  int st = launch_static_operand(a.act, a.act_kind == kActBf16, a.act_scale, act, row_scale, a.m, a.k, fragments,
+                                 a.stream);
   if (st) return st;
-  float *partial = p.part_bytes ? reinterpret_cast<float *>(ws + p.a_bytes + p.w_bytes) : nullptr;
+  LinearArgs b = a;
+  b.act_scale = row_scale;
+  if (fragments) return launch_gemm_skinny(b, act);
+  const GemmPlan p = plan_gemm(a.m, a.n, a.k);
   if (p.w_pre) {
-    const uint16_t *wbf = reinterpret_cast<const uint16_t *>(ws + p.a_bytes);
-    return launch_bf16_operands(a, p, abf, wbf, p.part_bytes ? p.splits : 1, partial);
+    const size_t chunks = size_t(a.n) * size_t(a.k) / 16;
+    decode_rows_kernel<<<unsigned(std::min<size_t>((chunks + 255) / 256, 4096)), 256, 0, a.stream>>>(
+        a.weight, reinterpret_cast<uint16_t *>(ws + p.a_bytes), chunks, nullptr, nullptr, 0);
+    if ((st = check_launch("hif8_static_linear (weight decode)"))) return st;
   }
-  return launch_plan<true>(a, p, abf, p.part_bytes ? p.splits : 1, partial);
+  return launch_prepared(b, p, ws);
 }
 
 size_t gemm_decoded_weight_workspace_size(int64_t m, int64_t n, int64_t k) {

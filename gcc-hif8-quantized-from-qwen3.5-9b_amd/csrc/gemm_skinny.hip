@@ -33,7 +33,7 @@
 // to zero, and the bf16 copy is zero-padded to a multiple of 64.
 #include <algorithm>
 
-#include "linear.h"
+#include "gemm_operand.h"
 
 namespace hif8 {
 namespace {
@@ -267,19 +267,21 @@ size_t skinny_workspace_size(int64_t m, int64_t k) {
   return size_t((m + 15) / 16 * 16) * size_t((k + kStepK - 1) / kStepK * kStepK) * 2;
 }
 
-int launch_gemm_skinny(const LinearArgs &a) {
+int launch_decode_fragments(const LinearArgs &a, uint16_t *act) {
   const int steps = int((a.k + kStepK - 1) / kStepK);
-  uint16_t *act = static_cast<uint16_t *>(a.workspace);
   const uint8_t *codes = static_cast<const uint8_t *>(a.act);
   const int64_t items = (a.m + 15) / 16 * steps * kWave;
   const unsigned blocks = unsigned(std::min<int64_t>((items + 255) / 256, 4096));
+  u32x4 *out = reinterpret_cast<u32x4 *>(act);
   if (a.k % 16 == 0 && aligned(codes, 16))
-    decode_fragments_kernel<true><<<blocks, 256, 0, a.stream>>>(codes, reinterpret_cast<u32x4 *>(act), int(a.m),
-                                                                int(a.k), steps);
+    decode_fragments_kernel<true><<<blocks, 256, 0, a.stream>>>(codes, out, int(a.m), int(a.k), steps);
   else
-    decode_fragments_kernel<false><<<blocks, 256, 0, a.stream>>>(codes, reinterpret_cast<u32x4 *>(act), int(a.m),
-                                                                 int(a.k), steps);
-  if (const int st = check_launch("soft_hif8 GEMM (activation decode)")) return st;
+    decode_fragments_kernel<false><<<blocks, 256, 0, a.stream>>>(codes, out, int(a.m), int(a.k), steps);
+  return check_launch("soft_hif8 GEMM (activation decode)");
+}
+
+int launch_gemm_skinny(const LinearArgs &a, const uint16_t *act) {
+  const int steps = int((a.k + kStepK - 1) / kStepK);
   // 32 weight rows per block share the activation fragments of a step (wide N,
   // or row tiles that fill the CUs); otherwise 16 give more CUs a block, and
   // eight wavefronts each a shorter chain.  MI355X, with the decode launch:

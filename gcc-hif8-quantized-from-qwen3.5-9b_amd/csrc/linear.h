@@ -77,10 +77,6 @@ size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k);
 // gemm_workspace_size, and for K % 64 != 0 the workspace with which the call
 // runs on the matrix cores (any smaller one: one thread per output).
 size_t gemm_scratch_size(int64_t m, int64_t n, int64_t k);
-// The GEMM of few rows, or of any K and alignment (gemm_skinny.hip); needs a
-// 256-byte aligned a.workspace of skinny_workspace_size(m, k) bytes.
-int launch_gemm_skinny(const LinearArgs &a);
-size_t skinny_workspace_size(int64_t m, int64_t k);
 // The GEMM with the weight already decoded to bf16 (a.weight_bf16; a.weight is
 // not read): the activation codes are decoded into the workspace and both
 // operands stream into LDS by DMA.  Needs k % 64 == 0, 16-byte aligned

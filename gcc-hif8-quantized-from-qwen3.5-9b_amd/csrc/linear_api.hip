@@ -1,7 +1,7 @@
 // C-ABI entry points of the soft HiF8 linear operators: validation mirrors
 // ValidateSoftLinear / SoftHif8StaticFusedGemm (hif8_native.cpp:241-316,784-861),
 // then M <= 4 goes to the GEMV kernel and larger M to the MFMA GEMM.
-#include "linear.h"
+#include "gemm_operand.h"
 
 using namespace hif8;
 
@@ -213,6 +213,33 @@ extern "C" int soft_hif8_static_fused_gemm(const void *x, int x_dtype, const uin
   a.act = x;
   a.act_kind = x_dtype == HIF8_DTYPE_BF16 ? kActBf16 : kActF16;
   return launch_gemv(a);
+}
+
+extern "C" size_t hif8_static_linear_workspace_size(int64_t m, int64_t n, int64_t k) {
+  return gemm_static_workspace_size(m, n, k);
+}
+
+extern "C" int hif8_static_linear(const void *x, int x_dtype, const uint8_t *weight, const float *fixed_scale,
+                                  const float *channel_scale, const void *bias, int bias_dtype, void *out,
+                                  int out_dtype, int64_t m, int64_t n, int64_t k, void *workspace,
+                                  size_t workspace_bytes, hif8_stream_t stream) {
+  clear_error();
+  int st = validate("hif8_static_linear", x, weight, fixed_scale, channel_scale, bias, bias_dtype, out, out_dtype, m,
+                    n, k);
+  if (st) return st;
+  if (!is_io_dtype(x_dtype))
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "activation must have dtype torch.float16 or torch.bfloat16");
+  const size_t need = gemm_static_workspace_size(m, n, k);
+  if (need == 0) return fail(HIF8_ERR_UNSUPPORTED, "hif8_static_linear requires M > 4 and K < 2^31 - 256");
+  if (!workspace || workspace_bytes < need || !aligned(workspace, 256))
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_static_linear: needs a 256-byte aligned workspace of %zu bytes", need);
+  LinearArgs a = codes_args(nullptr, weight, fixed_scale, channel_scale, bias, bias_dtype, out, out_dtype, m, n, k,
+                            stream);
+  a.act = x;
+  a.act_kind = x_dtype == HIF8_DTYPE_BF16 ? kActBf16 : kActF16;
+  a.workspace = workspace;
+  a.workspace_bytes = workspace_bytes;
+  return launch_gemm_static(a);
 }
 
 extern "C" int soft_hif8_fused_gemm(const void *x, int x_dtype, const uint8_t *weight,

@@ -357,6 +357,60 @@ at::Tensor SoftHif8StaticFusedGemm(const at::Tensor &activation, const at::Tenso
 }
 
 // hif8_native.cpp:671-782 (SoftHif8FusedGemm): dynamic per-row scale, M <= 2.
+// hif8_static_quant (one fixed scale) and soft_hif8_gemm in one call for M > 4:
+// the operand checks of both, the codes not materialised.
+at::Tensor Hif8StaticLinear(const at::Tensor &x, const at::Tensor &weight, const at::Tensor &fixed_scale,
+                            const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
+                            at::ScalarType output_dtype) {
+  CheckDeviceTensor(x, "x");
+  CheckDeviceTensor(weight, "weight");
+  CheckDeviceTensor(fixed_scale, "fixed_scale");
+  CheckDeviceTensor(channel_scale, "channel_scale");
+  TORCH_CHECK(x.scalar_type() == at::ScalarType::Half || x.scalar_type() == at::ScalarType::BFloat16,
+              "x must have dtype torch.float16 or torch.bfloat16");
+  TORCH_CHECK(weight.scalar_type() == at::ScalarType::Byte, "weight must have dtype torch.uint8");
+  TORCH_CHECK(fixed_scale.scalar_type() == at::ScalarType::Float, "fixed_scale must have dtype torch.float32");
+  TORCH_CHECK(channel_scale.scalar_type() == at::ScalarType::Float, "channel_scale must have dtype torch.float32");
+  TORCH_CHECK(x.dim() == 2, "x must have shape [M, K]");
+  TORCH_CHECK(weight.dim() == 2, "weight must have shape [N, K]");
+  TORCH_CHECK(fixed_scale.dim() == 1 && fixed_scale.numel() == 1, "fixed_scale must have shape [1]");
+  TORCH_CHECK(channel_scale.dim() == 1, "channel_scale must have shape [N]");
+  CheckPositiveDimensions(x, "x");
+  CheckPositiveDimensions(weight, "weight");
+  const int64_t m = x.size(0), k = x.size(1), n = weight.size(0);
+  TORCH_CHECK(m > 4, "hif8_static_linear requires M > 4");
+  TORCH_CHECK(weight.size(1) == k, "x and weight K dimensions differ: ", k, " != ", weight.size(1));
+  TORCH_CHECK(channel_scale.numel() == n, "channel_scale must contain one value per output channel");
+  CheckFitsUint32(m, "M");
+  CheckFitsUint32(n, "N");
+  CheckFitsUint32(k, "K");
+  const auto device = x.device();
+  CheckSameDevice(weight, device, "weight");
+  CheckSameDevice(fixed_scale, device, "fixed_scale");
+  CheckSameDevice(channel_scale, device, "channel_scale");
+  if (bias.has_value()) {
+    CheckDeviceTensor(*bias, "bias");
+    CheckSameDevice(*bias, device, "bias");
+    TORCH_CHECK(bias->dim() == 1, "bias must have shape [N]");
+    TORCH_CHECK(bias->numel() == n, "bias must contain N values");
+    TORCH_CHECK(bias->scalar_type() == at::ScalarType::Half || bias->scalar_type() == at::ScalarType::BFloat16,
+                "bias must have dtype torch.float16 or torch.bfloat16");
+  }
+  TORCH_CHECK(output_dtype == at::ScalarType::Half || output_dtype == at::ScalarType::BFloat16,
+              "output_dtype must be torch.float16 or torch.bfloat16");
+  const c10::OptionalDeviceGuard guard(device);
+  auto out = at::empty({m, n}, x.options().dtype(output_dtype));
+  const size_t ws_bytes = hif8_static_linear_workspace_size(m, n, k);
+  auto ws = at::empty({int64_t(ws_bytes)}, x.options().dtype(at::ScalarType::Byte));
+  CheckStatus(hif8_static_linear(x.data_ptr(), DtypeCode(x.scalar_type()), weight.data_ptr<uint8_t>(),
+                                 fixed_scale.data_ptr<float>(), channel_scale.data_ptr<float>(),
+                                 bias.has_value() ? bias->data_ptr() : nullptr,
+                                 bias.has_value() ? DtypeCode(bias->scalar_type()) : HIF8_DTYPE_NONE, out.data_ptr(),
+                                 DtypeCode(output_dtype), m, n, k, ws.data_ptr(), ws_bytes, CurrentStream(device)),
+              "hif8_static_linear");
+  return out;
+}
+
 at::Tensor SoftHif8FusedGemm(const at::Tensor &activation, const at::Tensor &weight,
                              const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
                              at::ScalarType output_dtype) {
@@ -1140,6 +1194,7 @@ TORCH_LIBRARY(vllm_ascend_hif8, m) {
   m.def("soft_hif8_gemv(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor? bias, ScalarType output_dtype) -> Tensor");
   m.def("soft_hif8_gemm(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor? bias, ScalarType output_dtype) -> Tensor");
   m.def("soft_hif8_static_fused_gemm(Tensor activation, Tensor weight, Tensor fixed_scale, Tensor channel_scale, Tensor? bias, ScalarType output_dtype) -> Tensor");
+  m.def("hif8_static_linear(Tensor x, Tensor weight, Tensor fixed_scale, Tensor channel_scale, Tensor? bias, ScalarType output_dtype) -> Tensor");
   m.def("hif8_kv_cache_write(Tensor key, Tensor value, Tensor(a!) key_cache, Tensor(b!) value_cache, Tensor slot_mapping, Tensor key_scale, Tensor value_scale, Tensor(c!)? invalid_slots=None) -> ()");
   m.def("hif8_paged_decode_attention(Tensor query, Tensor key_cache, Tensor value_cache, Tensor block_table, Tensor seq_lens, float scale, int max_seq_len) -> Tensor");
   m.def("hif8_paged_prefill_attention(Tensor query, Tensor key_cache, Tensor value_cache, Tensor block_table, Tensor query_start_loc, Tensor seq_lens, float scale, int max_query_len, int max_seq_len, bool causal=True) -> Tensor");
@@ -1169,6 +1224,7 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, CUDA, m) {
   m.impl("soft_hif8_gemv", &SoftHif8Gemv);
   m.impl("soft_hif8_gemm", &SoftHif8Gemm);
   m.impl("soft_hif8_static_fused_gemm", &SoftHif8StaticFusedGemm);
+  m.impl("hif8_static_linear", &Hif8StaticLinear);
   m.impl("hif8_kv_cache_write", &Hif8KVCacheWrite);
   m.impl("hif8_paged_decode_attention", &Hif8PagedDecodeAttention);
   m.impl("hif8_paged_prefill_attention", &Hif8PagedPrefillAttention);
@@ -1197,6 +1253,7 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, Meta, m) {
   m.impl("soft_hif8_gemv", &LinearMeta);
   m.impl("soft_hif8_gemm", &LinearMeta);
   m.impl("soft_hif8_static_fused_gemm", &LinearMeta);
+  m.impl("hif8_static_linear", &LinearMeta);
   m.impl("hif8_kv_cache_write", &Hif8KVCacheWriteMeta);
   m.impl("hif8_paged_decode_attention", &Hif8PagedDecodeAttentionMeta);
   m.impl("hif8_paged_prefill_attention", &Hif8PagedPrefillAttentionMeta);

@@ -26,7 +26,8 @@ LIB_NAME = "libhif8_rocm.so"
 ARCH = os.environ.get("HIF8_OFFLOAD_ARCH", "gfx950")
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 
-HIP_SOURCES = ["capi.hip", "static_quant.hip", "gemv.hip", "gemm.hip", "gemm_skinny.hip", "linear_api.hip", "kv_cache.hip",
+HIP_SOURCES = ["capi.hip", "static_quant.hip", "gemv.hip", "gemm.hip", "gemm_skinny.hip",
+               "static_operand.hip", "linear_api.hip", "kv_cache.hip",
                "embedding.hip", "model_ops.hip", "gdn_prefill.hip", "prefill_attention.hip"]
 
 HIPCC_FLAGS = [

@@ -354,6 +354,44 @@ def soft_static_fused_linear(
     return output.reshape(*x.shape[:-1], weight.shape[0])
 
 
+def static_linear(
+    x: "torch.Tensor",
+    weight: "torch.Tensor",
+    fixed_scale: "torch.Tensor",
+    weight_scale: "torch.Tensor",
+    bias: "torch.Tensor | None" = None,
+    *,
+    output_dtype: "torch.dtype",
+) -> "torch.Tensor":
+    """``soft_linear`` of ``static_quant(x, fixed_scale)`` for more than four
+    token rows and one fixed scale: equal outputs bit for bit, the codes in
+    between not materialised.  No counterpart in the reference."""
+    import torch
+
+    if x.dtype not in (torch.float16, torch.bfloat16):
+        raise TypeError(f"static HiFloat8 quant requires FP16/BF16 input, got {x.dtype}")
+    if fixed_scale.dtype != torch.float32 or fixed_scale.ndim != 1 or fixed_scale.numel() != 1:
+        raise TypeError("fixed_scale must be a 1D torch.float32 tensor of one value")
+    if fixed_scale.device != x.device:
+        raise ValueError(f"fixed_scale must be on {x.device}, got {fixed_scale.device}")
+    if weight.dtype != torch.uint8:
+        raise TypeError("soft HiFloat8 linear requires uint8 activation and weight tensors")
+    if x.ndim < 2 or weight.ndim != 2:
+        raise ValueError("activation must be at least 2D and weight must be 2D")
+    if x.shape[-1] != weight.shape[-1]:
+        raise ValueError(f"incompatible K dimensions: activation={x.shape[-1]}, weight={weight.shape[-1]}")
+    if weight_scale.dtype != torch.float32:
+        raise TypeError("soft HiFloat8 linear requires float32 activation and weight scales")
+    extension = load_extension()
+    flattened = _as_native_operand(x.reshape(-1, x.shape[-1]))
+    channel_scale = _as_native_operand(weight_scale.reshape(-1))
+    if channel_scale.numel() != weight.shape[0]:
+        raise ValueError("weight_scale must contain one value per output channel")
+    output = _operator("hif8_static_linear", extension)(
+        flattened, weight, _as_native_operand(fixed_scale), channel_scale, bias, output_dtype)
+    return output.reshape(*x.shape[:-1], weight.shape[0])
+
+
 def _validate_quantized_activation(source, data, scale, *, operation: str) -> None:
     """Post-conditions on a quantizer's outputs (native.py:287-304)."""
     import torch

@@ -210,6 +210,18 @@ int soft_hif8_static_fused_gemm(const void *x, int x_dtype, const uint8_t *weigh
                                 int64_t m, int64_t n, int64_t k, hif8_stream_t stream);
 
 /*
+ * hif8_static_quant with one fixed scale, then soft_hif8_gemm, for M > 4: the same
+ * outputs bit for bit, the activation encoded and decoded into the GEMM's bf16
+ * operand by one launch (the codes are not stored).  Needs a 256-byte aligned
+ * workspace of hif8_static_linear_workspace_size(m, n, k) bytes (0: not for M <= 4).
+ */
+size_t hif8_static_linear_workspace_size(int64_t m, int64_t n, int64_t k);
+int hif8_static_linear(const void *x, int x_dtype, const uint8_t *weight, const float *fixed_scale,
+                       const float *channel_scale, const void *bias, int bias_dtype, void *out, int out_dtype,
+                       int64_t m, int64_t n, int64_t k, void *workspace, size_t workspace_bytes,
+                       hif8_stream_t stream);
+
+/*
  * Dynamic-scale fused quant + GEMM for M <= 2 (the legacy soft scheme's
  * HIF8_SOFT_FUSED_GENERATION path).
  * Replaces aclnnSoftHif8FusedGemm as called by SoftHif8FusedGemm

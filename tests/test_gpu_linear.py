@@ -136,6 +136,37 @@ def test_few_row_and_ragged_gemm(native_ops, device, rows, channels, k):
     _check(y[:, torch.from_numpy(keep).to(device)], want)
 
 
+@pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,channels,k", [
+    # fragments (whole and partial steps, rows short of a tile), 128- and 256-row
+    # tiles with and without a K split, and the weight decoded once per call
+    (5, 40, 64), (17, 33, 100), (64, 4200, 1040), (70, 2100, 333), (129, 136, 12288), (300, 1000, 2048),
+    (512, 2048, 4096), (2048, 256, 1024),
+])
+def test_static_linear_equals_quant_then_gemm(native_ops, device, rows, channels, k, xdtype):
+    from hif8_rocm import native
+
+    g = torch.Generator().manual_seed(rows + k)
+    scale = torch.tensor([0.0009765625 * 1.1])
+    x = (torch.randn(rows, k, generator=g) * 3).to(xdtype)
+    # Quotients on and next to rounding boundaries, saturation, both zeros, tiny
+    # values, and one row each of Inf and NaN.
+    edge = (torch.tensor([1.0625, 1.125, 3.875, 17.0, 1.25 * 2 ** 15, 2.0 ** 17, 0.0, -0.0, 2.0 ** -23]) * scale)
+    x[0, :9] = edge.to(xdtype)
+    x[1, 3] = float("inf")
+    x[2, k - 1] = float("nan")
+    w = _t(random_codes((channels, k), seed=channels), device)
+    ws = (torch.rand(channels, generator=g) + 0.5).to(device)
+    bias = torch.randn(channels, generator=g).to(xdtype).to(device)
+    x, scale = x.to(device), scale.to(device)
+    codes, row_scale = native.static_quant(x, scale)
+    for b in (None, bias):
+        want = native.soft_linear(codes, w, row_scale, ws, b, output_dtype=xdtype)
+        got = native.static_linear(x, w, scale, ws, b, output_dtype=xdtype)
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("m", [1, 4])
 @pytest.mark.parametrize("n,k", LAYER_SHAPES)
 def test_decode_gemv_config_shapes(native_ops, device, m, n, k):
