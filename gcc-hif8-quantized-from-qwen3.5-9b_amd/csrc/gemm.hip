@@ -482,18 +482,30 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_kernel(
 // MFMAs: left to itself the compiler reads each fragment right before its
 // first MFMA and waits for it there).  One barrier per step, between the two
 // slices: after it the step's stage may be overwritten (the copy of step
-// kt + 2 is issued right there) and the next step's tile has landed, so the
+// kt + kStages is issued right there) and the next step's tile has landed, so the
 // second slice's MFMAs run while the next step's first fragments are read.
 // Wave sub-tiles are kBM / kWavesM rows x kBN / kWavesN columns: each A
 // fragment feeds kTN MFMAs in a row.
 //
-// kWDec: W is the uint8 code matrix, decoded in the kernel.  Each thread
-// loads 16-byte code chunks of the W tile a step ahead into VGPRs; during the
-// first slice of step kt it looks the codes of tile kt + 1 up in the 256-entry
-// bf16 table (LDS address 0) and stores them into that tile's stage (free
-// since the barrier of step kt - 1), lookups and the packing of their results
-// a few MFMAs apart, then loads the codes of tile kt + 2.  The A tile still
-// comes by DMA.
+// kWDec: W is the uint8 code matrix, decoded in the kernel.  Its code tiles come
+// by DMA into a ring of three LDS stages, four steps ahead; every thread reads
+// its chunks of a tile in the second slice of the step before it decodes them,
+// and during the first slice of step kt looks the codes of tile kt + 1 up in the
+// 256-entry bf16 table (LDS address 0) and stores them into that tile's stage
+// (free since the barrier of step kt - 1), lookups and the packing of their
+// results a few MFMAs apart.  Codes loaded into VGPRs instead made the compiler
+// wait for them with a count that knows nothing of the copies in flight, i.e.
+// for these too (MI355X: 512 x 4096 x 12288 in four splits 75.6 -> 72.3 us,
+// 256 x 4096 x 12288 48.8 -> 45.9, an unsplit 512 x 12288 x 4096 75.9 -> 69.9).
+// What bounds it now is LDS: per step of a 256 x 128 block 1024 clocks of
+// fragment reads, ~500 of lookups and ~500 of copies and stores.
+//
+// kStages K steps of both tiles sit in LDS: three where they fit beside the
+// table and the code ring, so that a copy has two steps to land in, else two.
+constexpr int dma_stages(int bm, int bn, bool wdec) {
+  return 3 * (bm + bn) * kBK * 2 + (wdec ? 3 * bn * kBK : 0) + 512 <= 160 * 1024 ? 3 : 2;
+}
+
 template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec>
 __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
     const uint16_t *__restrict__ A, const float *__restrict__ ts, const void *__restrict__ Wv,
@@ -509,6 +521,11 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
   static_assert(kDmaA * kWaves * 1024 == int(kStageA) && (kWDec || kDmaB * kWaves * 1024 == int(kStageB)),
                 "tile copies split evenly over the waves");
   constexpr int kDec = kWDec ? kBN * kBK / 8 / kT : 0;  // 8-code W chunks per thread and step
+  constexpr int kStages = dma_stages(kBM, kBN, kWDec);
+  // 1 KiB copies of a code tile (16 rows of 64 codes each) and their number per
+  // wave; the last ones repeat where they do not divide over the waves.
+  constexpr int kCodeCopies = kBN * kBK / 1024, kDmaC = kWDec ? (kCodeCopies + kWaves - 1) / kWaves : 0;
+  constexpr int kCopies = kDmaA + kDmaB;
   static_assert(!kWDec || kDec * 8 * kT == kBN * kBK, "W decode split evenly over the threads");
   const uint16_t *W = static_cast<const uint16_t *>(Wv);
   const uint8_t *Wc = static_cast<const uint8_t *>(Wv);
@@ -550,23 +567,33 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
   const uint16_t *a_split = A + size_t(m0) * K + k_first, *w_split = W + size_t(n0) * K + k_first;
   const uint32_t lds0 = lds_address(smem);
 
-  // W codes (kWDec): chunk c of this thread is q = tid + c * kT of the tile,
-  // row q / 8, codes 8 (q % 8) .. 8 (q % 8) + 7 of the step's 64, which
-  // decode to granule q % 8 of the row.
-  uint32_t wco[kDec > 0 ? kDec : 1], wdst[kDec > 0 ? kDec : 1];
+  // W codes (kWDec): copy j of this wave brings 1 KiB q = (wave + kWaves j) %
+  // kCodeCopies of the tile's codes (rows 16 q .. 16 q + 15, lane i the piece
+  // i % 4 of row i / 4) into a ring of three code stages.  Chunk c of this
+  // thread is q = tid + c * kT of the tile, row q / 8, codes 8 (q % 8) ..
+  // 8 (q % 8) + 7 of the step's 64, which decode to granule q % 8 of the row.
+  constexpr uint32_t kCodeStage = kWDec ? kBN * kBK : 0, kCodes = kStages * kStage;
+  uint32_t oc[kDmaC > 0 ? kDmaC : 1], wdst[kDec > 0 ? kDec : 1];
   uint2 wq[kDec > 0 ? kDec : 1];
   if constexpr (kWDec) {
 #pragma unroll
+    for (int j = 0; j < kDmaC; ++j) {
+      const int r = 16 * ((wave + kWaves * j) % kCodeCopies) + (lane >> 2);
+      oc[j] = uint32_t(min(n0 + r, N - 1) - n0) * uint32_t(K) + uint32_t(lane & 3) * 16u;
+    }
+#pragma unroll
     for (int c = 0; c < kDec; ++c) {
       const int q = tid + c * kT, r = q >> 3, gq = q & 7;
-      wco[c] = uint32_t(min(n0 + r, N - 1) - n0) * uint32_t(K) + uint32_t(gq) * 8u;
       wdst[c] = kStageA + uint32_t(r) * 128u + uint32_t((gq ^ (r & 7)) * 16);
     }
   }
   const uint8_t *wc_split = Wc + size_t(n0) * K + k_first;
-  auto load_codes = [&](int kt) {
-#pragma unroll
-    for (int c = 0; c < kDec; ++c) wq[c] = *reinterpret_cast<const uint2 *>(wc_split + size_t(kt) * kBK + wco[c]);
+  auto copy_codes = [&](int kt, int ring, int j) {
+    dma16_offset(wc_split + size_t(kt) * kBK, oc[j],
+                 lds0 + kCodes + uint32_t(ring) * kCodeStage + uint32_t((wave + kWaves * j) % kCodeCopies) * 1024u);
+  };
+  auto read_codes = [&](int ring, int c) {
+    wq[c] = *reinterpret_cast<const uint2 *>(smem + kCodes + uint32_t(ring) * kCodeStage + uint32_t(tid + c * kT) * 8u);
   };
   // Chunk c: looks up its 8 codes (8 table entries), then packs them into
   // its bf16 granule in the stage at `stage`.
@@ -613,27 +640,26 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
 
   // One 32-wide slice, its order pinned by scheduling barriers: the MFMAs of
   // (fa, fb); after every kPerRead of them one read of the next slice's
-  // fragments (into na, nb, from stage `next`, granule offset g); and, with
-  // kCopy, one of this wave's copies of step copy_kt into stage copy_stage
-  // after every kCopyEvery MFMAs (spread over the slice; issuing them
-  // together at its start measured the same).
-  constexpr int kCopies = kDmaA + kDmaB;
+  // fragments (into na, nb, from stage `next`, granule offset g).  Second
+  // slices (kSecond) also issue this wave's copies of step copy_kt into stage
+  // copy_stage after every kCopyEvery MFMAs (spread over the slice; issuing them
+  // together at its start measured the same) and, with kWDec, read the codes of
+  // tile kt + 2 (ring stage code_from) and copy those of tile code_kt into ring
+  // stage code_to last; first slices decode tile kt + 1 into dec_stage.
   constexpr int kCopyEvery = kMfmas / kCopies > 0 ? kMfmas / kCopies : 1;
   // Decode positions (kWDec, first slice of a step): the lookups of chunk c
-  // after MFMA c * kDecStep, its packing and store kDecGap MFMAs later; the
-  // next codes' loads after the last store.
+  // after MFMA c * kDecStep, its packing and store kDecGap MFMAs later.
   constexpr int kDecStep = kDec > 0 ? (kMfmas * 3 / 4) / kDec : 1;
   constexpr int kDecGap = kDecStep / 2 > 0 ? kDecStep / 2 : 1;
-  static_assert(!kWDec || (kDecGap <= kDecStep && (kDec - 1) * kDecStep + kDecGap + 1 < kMfmas),
-                "each chunk packed before the next lookups; the next codes loaded within the slice");
-  auto slice = [&](auto do_read, auto do_copy, auto do_decode, const bf16x8_t (&fa)[kTM],
-                   const bf16x8_t (&fb)[kTN], bf16x8_t (&na)[kTM], bf16x8_t (&nb)[kTN], const uint8_t *next,
-                   uint32_t g, int copy_kt, int copy_stage, uint8_t *dec_stage, int codes_kt) {
-    constexpr bool kRead = decltype(do_read)::value, kCopy = decltype(do_copy)::value;
+  static_assert(!kWDec || (kDecGap <= kDecStep && (kDec - 1) * kDecStep + kDecGap < kMfmas && kDec <= kMfmas),
+                "each chunk packed before the next lookups, within the slice");
+  auto slice = [&](auto do_read, auto second, auto do_decode, const bf16x8_t (&fa)[kTM], const bf16x8_t (&fb)[kTN],
+                   bf16x8_t (&na)[kTM], bf16x8_t (&nb)[kTN], const uint8_t *next, uint32_t g, int copy_kt,
+                   int copy_stage, uint8_t *dec_stage, int code_kt, int code_to, int code_from) {
+    constexpr bool kRead = decltype(do_read)::value, kSecond = decltype(second)::value;
     constexpr bool kDecode = decltype(do_decode)::value;
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + uint32_t(copy_stage) * kStage);
     const uint16_t *sa = a_split + size_t(copy_kt) * kBK, *sw = w_split + size_t(copy_kt) * kBK;
-    if constexpr (kDecode) wait_vmcnt<kDmaA>();  // this step's codes (the A copy issued after them may fly on)
 #pragma unroll
     for (int p = 0; p < kMfmas; ++p) {
       acc[p / kTN][p % kTN] =
@@ -648,13 +674,16 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
                 __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4 *>(next + rb + (r - kTM) * 2048 + g));
         }
       }
-      if constexpr (kCopy) {
+      if constexpr (kSecond) {
         if (p % kCopyEvery == 0 && p / kCopyEvery < kCopies) {
           const int d = p / kCopyEvery;
           if (d < kDmaA)
             dma16_offset(sa, oa[d], dst + uint32_t(wave * kDmaA + d) * 1024u);
           else
             dma16_offset(sw, ob[d - kDmaA], dst + kStageA + uint32_t(wave * kDmaB + d - kDmaA) * 1024u);
+        }
+        if constexpr (kWDec) {
+          if (p < kDec) read_codes(code_from, p);
         }
       }
       if constexpr (kDecode) {
@@ -663,62 +692,83 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
         if (p >= kDecGap && (p - kDecGap) % kDecStep == 0 && (p - kDecGap) / kDecStep < kDec)
           pack_store((p - kDecGap) / kDecStep, dec_stage);
         if (p % kDecStep == 0 && p / kDecStep < kDec) lookup(p / kDecStep);
-        if (p == (kDec - 1) * kDecStep + kDecGap + 1) load_codes(codes_kt);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (kSecond && kWDec) {
+#pragma unroll
+      for (int j = 0; j < kDmaC; ++j) copy_codes(code_kt, code_to, j);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
   const std::true_type yes;
   const std::false_type no;
 
+
   // The loop body is free of branches (a branch there splits the
   // accumulators' live ranges into copies): the last step runs after it, and
-  // the copy that the second-to-last step would issue for step KT repeats
-  // step KT - 1 into the stage nobody reads any more.
+  // the copies that the steps before it would issue past step KT - 1 repeat
+  // that one into stages nobody reads any more.
   const int KT = ksteps;
+  auto last = [&](int kt) { return min(kt, KT - 1); };
   if constexpr (kWDec) {
-    // Tile 0: codes and A copy; its codes decoded here (one code buffer, so
-    // tile 1's codes are loaded after), then tile 1's codes and A copy.
-    load_codes(0);
+    // Tile 0's A copy and codes, decoded here; tile 1's codes into registers;
+    // then the copies of the next tiles in the order the loop counts on.
     copy(0, 0);
-    wait_vmcnt<kDmaA>();
-    lds_barrier();  // the table
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < kDmaC; ++j) copy_codes(last(t), t, j);
+    wait_vmcnt<0>();
+    lds_barrier();  // ... and the table
 #pragma unroll
     for (int c = 0; c < kDec; ++c) {
+      read_codes(0, c);
       lookup(c);
       pack_store(c, smem);
     }
-    load_codes(min(1, KT - 1));
-    copy(min(1, KT - 1), 1);
-    wait_vmcnt<kDmaA + kDec>();  // tile 0's A copy
+#pragma unroll
+    for (int c = 0; c < kDec; ++c) read_codes(1, c);
+    lds_barrier();  // tile 0 complete, ring stages 0 and 1 read
+    if constexpr (kStages == 3) copy(last(1), 1);
+#pragma unroll
+    for (int j = 0; j < kDmaC; ++j) copy_codes(last(2), 2, j);
+    copy(last(kStages - 1), kStages - 1);
+#pragma unroll
+    for (int j = 0; j < kDmaC; ++j) copy_codes(last(3), 0, j);
   } else {
     copy(0, 0);
-    if (KT > 1) {
-      copy(1, 1);
-      wait_vmcnt<kDmaA + kDmaB>();
-    } else {
-      wait_vmcnt<0>();
-    }
+#pragma unroll
+    for (int t = 1; t < kStages; ++t) copy(last(t), t);
+    wait_vmcnt<(kStages - 1) * kCopies>();
+    lds_barrier();
   }
-  lds_barrier();
   read(fa0, fb0, smem, g0);
+  // Stages of steps kt and kt + 1; ring stages of the codes of tiles kt + 1
+  // (in registers, so tile kt + 4's go there) and kt + 2.
+  int cur = 0, next = 1, ring = 1, ring_next = 2;
   for (int kt = 0; kt + 1 < KT; ++kt) {
     // Slice 0 of step kt (registers 0) while slice 1 is read (registers 1)
     // and (kWDec) the codes of tile kt + 1 are decoded into its stage.
-    slice(yes, no, std::integral_constant<bool, kWDec>{}, fa0, fb0, fa1, fb1, smem + (kt & 1) * kStage, g1, 0, 0,
-          smem + ((kt + 1) & 1) * kStage, min(kt + 2, KT - 1));
-    // This wave's copy of step kt + 1 has landed (and its stores of the
-    // decoded W) and its reads of stage kt & 1 are done; after the barrier
-    // the same holds for every wave.  The codes of tile kt + 2 may fly on.
-    wait_vmcnt<kDec>();
+    slice(yes, no, std::integral_constant<bool, kWDec>{}, fa0, fb0, fa1, fb1, smem + cur * kStage, g1, 0, 0,
+          smem + next * kStage, 0, 0, 0);
+    // This wave's copies of step kt + 1 and of the codes of tile kt + 2 have
+    // landed (and its stores of the decoded W) and its reads of step kt's stage
+    // are done; after the barrier the same holds for every wave.  The newest
+    // codes, and with three stages the newest tile copy, may fly on.
+    wait_vmcnt<(kStages - 2) * kCopies + kDmaC>();
     lds_barrier();
     // Slice 1 of step kt while slice 0 of step kt + 1 is read and step
-    // kt + 2 is copied into the stage step kt used.
-    slice(yes, yes, no, fa1, fb1, fa0, fb0, smem + ((kt + 1) & 1) * kStage, g0, min(kt + 2, KT - 1), kt & 1, smem,
-          0);
+    // kt + kStages is copied into the stage step kt used.
+    slice(yes, yes, no, fa1, fb1, fa0, fb0, smem + next * kStage, g0, last(kt + kStages), cur, smem, last(kt + 4),
+          ring, ring_next);
+    cur = next;
+    next = next + 1 == kStages ? 0 : next + 1;
+    ring = ring_next;
+    ring_next = ring_next == 2 ? 0 : ring_next + 1;
   }
-  slice(yes, no, no, fa0, fb0, fa1, fb1, smem + ((KT - 1) & 1) * kStage, g1, 0, 0, smem, 0);
-  slice(no, no, no, fa1, fb1, fa0, fb0, smem, g0, 0, 0, smem, 0);
+  slice(yes, no, no, fa0, fb0, fa1, fb1, smem + cur * kStage, g1, 0, 0, smem, 0, 0, 0);
+  slice(no, no, no, fa1, fb1, fa0, fb0, smem, g0, 0, 0, smem, 0, 0, 0);
   wait_vmcnt<0>();  // the repeated copy (and codes) of the last step
 
   if (partial) {
@@ -922,6 +972,14 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int64_t k, bool decoded_weight = false)
       p.splits = s128;
     }
   }
+  // ... and unsplit where the 128-tiles would be, at one to two per CU: the
+  // 256 x 128 blocks decode each weight tile half as often (MI355X, 512 x 12288
+  // x 4096 93.8 -> 69.9 us, 256 x 24576 x 4096 93.1 -> 69.6; sums unchanged).
+  if (!decoded_weight && wdec128_env && tile_env == 0 && split_env == 0 && m >= 256 && k < kMaxDmaK &&
+      k % kBK == 0 && p.tile == 128 && p.splits == 1 && tiles > 256 && tiles256x128 <= 256) {
+    p.tile = 256;
+    p.bn = 128;
+  }
   p.w_pre = false;
   p.a_bytes = (size_t(m) * size_t(k) * 2 + 255) / 256 * 256;
   p.w_bytes = p.w_pre ? (size_t(n) * size_t(k) * 2 + 255) / 256 * 256 : 0;
@@ -955,7 +1013,8 @@ int launch_tiled(const LinearArgs &a, const void *act, const void *wt, int split
 // is the bf16 weight, or (kWDec) the codes.
 template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec = false>
 int launch_dma(const LinearArgs &a, const uint16_t *act, const void *wt, int splits, float *partial) {
-  constexpr size_t kSmem = std::max<size_t>(2 * size_t(kBM + kBN) * kBK * 2,
+  constexpr size_t kSmem = std::max<size_t>(dma_stages(kBM, kBN, kWDec) * size_t(kBM + kBN) * kBK * 2 +
+                                                (kWDec ? 3 * size_t(kBN) * kBK : 0),
                                             size_t(kWavesM * kWavesN) *
                                                 epilogue_region_bytes<kBM / kWavesM / 16, kBN / kWavesN / 16>());
   constexpr int kT = kWave * kWavesM * kWavesN;

@@ -136,6 +136,21 @@ def test_few_row_and_ragged_gemm(native_ops, device, rows, channels, k):
     _check(y[:, torch.from_numpy(keep).to(device)], want)
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("rows,channels", [(300, 11001), (500, 22024)])
+def test_weight_decoding_tiles_of_few_steps(native_ops, device, rows, channels, k):
+    """The 256-row blocks that decode the weight in the kernel (256 x 128 unsplit;
+    256 x 192), with fewer K steps than their pipeline is deep and ragged edges."""
+    a = random_codes((rows, k), seed=rows + k)
+    w = random_codes((channels, k), seed=channels + k)
+    ts = np.linspace(1e-3, 2e-3, rows, dtype=np.float32)
+    cs = np.linspace(1e-3, 2e-3, channels, dtype=np.float32)
+    want = o.linear_u8_u8(a, ts, w, cs, None)
+    y = native_ops.soft_hif8_gemm(_t(a, device), _t(w, device), _t(ts, device), _t(cs, device), None, torch.bfloat16)
+    torch.cuda.synchronize()
+    _check(y, want)
+
+
 @pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,channels,k", [
     # fragments (whole and partial steps, rows short of a tile), 128- and 256-row
