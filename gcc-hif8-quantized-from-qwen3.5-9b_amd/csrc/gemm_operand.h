@@ -19,8 +19,8 @@ int launch_decode_fragments(const LinearArgs &a, uint16_t *act);
 int launch_gemm_skinny(const LinearArgs &a, const uint16_t *act);
 
 // out = static_quant(x) W^T ...: a.act fp16 / bf16 x (a.act_kind kActF16 /
-// kActBf16), a.act_scale the fixed scale, m > 4; a 256-byte aligned
-// a.workspace of gemm_static_workspace_size(m, n, k) bytes (gemm.hip).
+// kActBf16), a.act_scale the fixed scale, m > 4 or k % 16 != 0; a 256-byte
+// aligned a.workspace of gemm_static_workspace_size(m, n, k) bytes (gemm.hip).
 int launch_gemm_static(const LinearArgs &a);
 size_t gemm_static_workspace_size(int64_t m, int64_t n, int64_t k);
 

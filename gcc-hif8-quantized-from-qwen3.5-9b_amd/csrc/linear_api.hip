@@ -144,6 +144,11 @@ extern "C" int soft_hif8_gemm_with_workspace(const uint8_t *activation, const ui
                             out_dtype, m, n, k, stream);
   a.workspace = workspace;
   a.workspace_bytes = workspace_bytes;
+  if (m <= 4 && workspace && gemm_scratch_size(m, n, k) && workspace_bytes >= gemm_scratch_size(m, n, k)) {
+    uint16_t *act = static_cast<uint16_t *>(workspace);
+    st = launch_decode_fragments(a, act);
+    return st ? st : launch_gemm_skinny(a, act);
+  }
   return m <= 4 ? launch_gemv(a) : launch_gemm(a);
 }
 
@@ -230,7 +235,7 @@ extern "C" int hif8_static_linear(const void *x, int x_dtype, const uint8_t *wei
   if (!is_io_dtype(x_dtype))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "activation must have dtype torch.float16 or torch.bfloat16");
   const size_t need = gemm_static_workspace_size(m, n, k);
-  if (need == 0) return fail(HIF8_ERR_UNSUPPORTED, "hif8_static_linear requires M > 4 and K < 2^31 - 256");
+  if (need == 0) return fail(HIF8_ERR_UNSUPPORTED, "hif8_static_linear requires M > 4 or K %% 16 != 0, and K < 2^31 - 256");
   if (!workspace || workspace_bytes < need || !aligned(workspace, 256))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_static_linear: needs a 256-byte aligned workspace of %zu bytes", need);
   LinearArgs a = codes_args(nullptr, weight, fixed_scale, channel_scale, bias, bias_dtype, out, out_dtype, m, n, k,

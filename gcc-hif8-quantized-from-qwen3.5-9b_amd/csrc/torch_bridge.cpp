@@ -184,9 +184,19 @@ at::Tensor Hif8ScaledDecode(const at::Tensor &data, const at::Tensor &scale) {
   return out;
 }
 
+at::Tensor SoftHif8Gemm(const at::Tensor &activation, const at::Tensor &weight, const at::Tensor &token_scale,
+                        const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
+                        at::ScalarType output_dtype);
+
 at::Tensor SoftHif8Gemv(const at::Tensor &activation, const at::Tensor &weight, const at::Tensor &token_scale,
                         const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
                         at::ScalarType output_dtype) {
+  if (activation.dim() == 2 && activation.size(1) % 16 != 0) {
+    // Rows the GEMV cannot stream in 16-byte chunks: the GEMM's few-row kernel,
+    // as soft_hif8_gemm runs them.
+    ValidateSoftLinear(activation, weight, token_scale, channel_scale, bias, output_dtype, true);
+    return SoftHif8Gemm(activation, weight, token_scale, channel_scale, bias, output_dtype);
+  }
   return SoftLinear(activation, weight, token_scale, channel_scale, bias, output_dtype, true, "soft_hif8_gemv",
                     &soft_hif8_gemv);
 }
@@ -248,6 +258,61 @@ at::Tensor Hif8DecodeBf16(const at::Tensor &codes) {
   return out;
 }
 
+// hif8_static_quant (one fixed scale) and soft_hif8_gemm in one call for M > 4
+// or K % 16 != 0:
+// the operand checks of both, the codes not materialised.
+at::Tensor Hif8StaticLinear(const at::Tensor &x, const at::Tensor &weight, const at::Tensor &fixed_scale,
+                            const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
+                            at::ScalarType output_dtype) {
+  CheckDeviceTensor(x, "x");
+  CheckDeviceTensor(weight, "weight");
+  CheckDeviceTensor(fixed_scale, "fixed_scale");
+  CheckDeviceTensor(channel_scale, "channel_scale");
+  TORCH_CHECK(x.scalar_type() == at::ScalarType::Half || x.scalar_type() == at::ScalarType::BFloat16,
+              "x must have dtype torch.float16 or torch.bfloat16");
+  TORCH_CHECK(weight.scalar_type() == at::ScalarType::Byte, "weight must have dtype torch.uint8");
+  TORCH_CHECK(fixed_scale.scalar_type() == at::ScalarType::Float, "fixed_scale must have dtype torch.float32");
+  TORCH_CHECK(channel_scale.scalar_type() == at::ScalarType::Float, "channel_scale must have dtype torch.float32");
+  TORCH_CHECK(x.dim() == 2, "x must have shape [M, K]");
+  TORCH_CHECK(weight.dim() == 2, "weight must have shape [N, K]");
+  TORCH_CHECK(fixed_scale.dim() == 1 && fixed_scale.numel() == 1, "fixed_scale must have shape [1]");
+  TORCH_CHECK(channel_scale.dim() == 1, "channel_scale must have shape [N]");
+  CheckPositiveDimensions(x, "x");
+  CheckPositiveDimensions(weight, "weight");
+  const int64_t m = x.size(0), k = x.size(1), n = weight.size(0);
+  TORCH_CHECK(m > 4 || k % 16 != 0, "hif8_static_linear requires M > 4 or K % 16 != 0");
+  TORCH_CHECK(weight.size(1) == k, "x and weight K dimensions differ: ", k, " != ", weight.size(1));
+  TORCH_CHECK(channel_scale.numel() == n, "channel_scale must contain one value per output channel");
+  CheckFitsUint32(m, "M");
+  CheckFitsUint32(n, "N");
+  CheckFitsUint32(k, "K");
+  const auto device = x.device();
+  CheckSameDevice(weight, device, "weight");
+  CheckSameDevice(fixed_scale, device, "fixed_scale");
+  CheckSameDevice(channel_scale, device, "channel_scale");
+  if (bias.has_value()) {
+    CheckDeviceTensor(*bias, "bias");
+    CheckSameDevice(*bias, device, "bias");
+    TORCH_CHECK(bias->dim() == 1, "bias must have shape [N]");
+    TORCH_CHECK(bias->numel() == n, "bias must contain N values");
+    TORCH_CHECK(bias->scalar_type() == at::ScalarType::Half || bias->scalar_type() == at::ScalarType::BFloat16,
+                "bias must have dtype torch.float16 or torch.bfloat16");
+  }
+  TORCH_CHECK(output_dtype == at::ScalarType::Half || output_dtype == at::ScalarType::BFloat16,
+              "output_dtype must be torch.float16 or torch.bfloat16");
+  const c10::OptionalDeviceGuard guard(device);
+  auto out = at::empty({m, n}, x.options().dtype(output_dtype));
+  const size_t ws_bytes = hif8_static_linear_workspace_size(m, n, k);
+  auto ws = at::empty({int64_t(ws_bytes)}, x.options().dtype(at::ScalarType::Byte));
+  CheckStatus(hif8_static_linear(x.data_ptr(), DtypeCode(x.scalar_type()), weight.data_ptr<uint8_t>(),
+                                 fixed_scale.data_ptr<float>(), channel_scale.data_ptr<float>(),
+                                 bias.has_value() ? bias->data_ptr() : nullptr,
+                                 bias.has_value() ? DtypeCode(bias->scalar_type()) : HIF8_DTYPE_NONE, out.data_ptr(),
+                                 DtypeCode(output_dtype), m, n, k, ws.data_ptr(), ws_bytes, CurrentStream(device)),
+              "hif8_static_linear");
+  return out;
+}
+
 at::Tensor SoftHif8StaticFusedGemm(const at::Tensor &activation, const at::Tensor &weight,
                                    const at::Tensor &fixed_scale, const at::Tensor &channel_scale,
                                    const c10::optional<at::Tensor> &bias, at::ScalarType output_dtype) {
@@ -287,6 +352,9 @@ at::Tensor SoftHif8StaticFusedGemm(const at::Tensor &activation, const at::Tenso
   }
   TORCH_CHECK(output_dtype == at::ScalarType::Half || output_dtype == at::ScalarType::BFloat16,
               "output_dtype must be torch.float16 or torch.bfloat16");
+  // Rows the GEMV cannot stream in 16-byte chunks run as more rows do.
+  if (activation.size(1) % 16 != 0)
+    return Hif8StaticLinear(activation, weight, fixed_scale, channel_scale, bias, output_dtype);
   const c10::OptionalDeviceGuard guard(device);
   auto out = at::empty({activation.size(0), weight.size(0)}, activation.options().dtype(output_dtype));
   const void *bias_ptr = bias.has_value() ? bias->data_ptr() : nullptr;
@@ -357,60 +425,6 @@ at::Tensor SoftHif8StaticFusedGemm(const at::Tensor &activation, const at::Tenso
 }
 
 // hif8_native.cpp:671-782 (SoftHif8FusedGemm): dynamic per-row scale, M <= 2.
-// hif8_static_quant (one fixed scale) and soft_hif8_gemm in one call for M > 4:
-// the operand checks of both, the codes not materialised.
-at::Tensor Hif8StaticLinear(const at::Tensor &x, const at::Tensor &weight, const at::Tensor &fixed_scale,
-                            const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
-                            at::ScalarType output_dtype) {
-  CheckDeviceTensor(x, "x");
-  CheckDeviceTensor(weight, "weight");
-  CheckDeviceTensor(fixed_scale, "fixed_scale");
-  CheckDeviceTensor(channel_scale, "channel_scale");
-  TORCH_CHECK(x.scalar_type() == at::ScalarType::Half || x.scalar_type() == at::ScalarType::BFloat16,
-              "x must have dtype torch.float16 or torch.bfloat16");
-  TORCH_CHECK(weight.scalar_type() == at::ScalarType::Byte, "weight must have dtype torch.uint8");
-  TORCH_CHECK(fixed_scale.scalar_type() == at::ScalarType::Float, "fixed_scale must have dtype torch.float32");
-  TORCH_CHECK(channel_scale.scalar_type() == at::ScalarType::Float, "channel_scale must have dtype torch.float32");
-  TORCH_CHECK(x.dim() == 2, "x must have shape [M, K]");
-  TORCH_CHECK(weight.dim() == 2, "weight must have shape [N, K]");
-  TORCH_CHECK(fixed_scale.dim() == 1 && fixed_scale.numel() == 1, "fixed_scale must have shape [1]");
-  TORCH_CHECK(channel_scale.dim() == 1, "channel_scale must have shape [N]");
-  CheckPositiveDimensions(x, "x");
-  CheckPositiveDimensions(weight, "weight");
-  const int64_t m = x.size(0), k = x.size(1), n = weight.size(0);
-  TORCH_CHECK(m > 4, "hif8_static_linear requires M > 4");
-  TORCH_CHECK(weight.size(1) == k, "x and weight K dimensions differ: ", k, " != ", weight.size(1));
-  TORCH_CHECK(channel_scale.numel() == n, "channel_scale must contain one value per output channel");
-  CheckFitsUint32(m, "M");
-  CheckFitsUint32(n, "N");
-  CheckFitsUint32(k, "K");
-  const auto device = x.device();
-  CheckSameDevice(weight, device, "weight");
-  CheckSameDevice(fixed_scale, device, "fixed_scale");
-  CheckSameDevice(channel_scale, device, "channel_scale");
-  if (bias.has_value()) {
-    CheckDeviceTensor(*bias, "bias");
-    CheckSameDevice(*bias, device, "bias");
-    TORCH_CHECK(bias->dim() == 1, "bias must have shape [N]");
-    TORCH_CHECK(bias->numel() == n, "bias must contain N values");
-    TORCH_CHECK(bias->scalar_type() == at::ScalarType::Half || bias->scalar_type() == at::ScalarType::BFloat16,
-                "bias must have dtype torch.float16 or torch.bfloat16");
-  }
-  TORCH_CHECK(output_dtype == at::ScalarType::Half || output_dtype == at::ScalarType::BFloat16,
-              "output_dtype must be torch.float16 or torch.bfloat16");
-  const c10::OptionalDeviceGuard guard(device);
-  auto out = at::empty({m, n}, x.options().dtype(output_dtype));
-  const size_t ws_bytes = hif8_static_linear_workspace_size(m, n, k);
-  auto ws = at::empty({int64_t(ws_bytes)}, x.options().dtype(at::ScalarType::Byte));
-  CheckStatus(hif8_static_linear(x.data_ptr(), DtypeCode(x.scalar_type()), weight.data_ptr<uint8_t>(),
-                                 fixed_scale.data_ptr<float>(), channel_scale.data_ptr<float>(),
-                                 bias.has_value() ? bias->data_ptr() : nullptr,
-                                 bias.has_value() ? DtypeCode(bias->scalar_type()) : HIF8_DTYPE_NONE, out.data_ptr(),
-                                 DtypeCode(output_dtype), m, n, k, ws.data_ptr(), ws_bytes, CurrentStream(device)),
-              "hif8_static_linear");
-  return out;
-}
-
 at::Tensor SoftHif8FusedGemm(const at::Tensor &activation, const at::Tensor &weight,
                              const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
                              at::ScalarType output_dtype) {

@@ -148,9 +148,9 @@ size_t soft_hif8_gemm_workspace_size(int64_t m, int64_t n, int64_t k);
 
 /*
  * The workspace with which soft_hif8_gemm_with_workspace runs fastest: the size
- * above, and for K that is no multiple of 64, where that is 0 and a call without
- * workspace computes one output per thread, the bf16 activation fragments with
- * which the call runs on the matrix cores.
+ * above, and for K that is no multiple of 64 (16 for M <= 4), where that is 0 and
+ * a call without workspace computes one output per thread or wavefront, the bf16
+ * activation fragments with which the call runs on the matrix cores.
  */
 size_t soft_hif8_gemm_scratch_size(int64_t m, int64_t n, int64_t k);
 
@@ -210,10 +210,11 @@ int soft_hif8_static_fused_gemm(const void *x, int x_dtype, const uint8_t *weigh
                                 int64_t m, int64_t n, int64_t k, hif8_stream_t stream);
 
 /*
- * hif8_static_quant with one fixed scale, then soft_hif8_gemm, for M > 4: the same
- * outputs bit for bit, the activation encoded and decoded into the GEMM's bf16
- * operand by one launch (the codes are not stored).  Needs a 256-byte aligned
- * workspace of hif8_static_linear_workspace_size(m, n, k) bytes (0: not for M <= 4).
+ * hif8_static_quant with one fixed scale, then soft_hif8_gemm with the workspace of
+ * soft_hif8_gemm_scratch_size, for M > 4 or K % 16 != 0: the same outputs bit for
+ * bit, the activation encoded and decoded into the GEMM's bf16 operand by one
+ * launch (the codes are not stored).  Needs a 256-byte aligned workspace of
+ * hif8_static_linear_workspace_size(m, n, k) bytes (0: sizes that the GEMV takes).
  */
 size_t hif8_static_linear_workspace_size(int64_t m, int64_t n, int64_t k);
 int hif8_static_linear(const void *x, int x_dtype, const uint8_t *weight, const float *fixed_scale,

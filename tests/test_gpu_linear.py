@@ -157,6 +157,8 @@ def test_weight_decoding_tiles_of_few_steps(native_ops, device, rows, channels, 
     # tiles with and without a K split, and the weight decoded once per call
     (5, 40, 64), (17, 33, 100), (64, 4200, 1040), (70, 2100, 333), (129, 136, 12288), (300, 1000, 2048),
     (512, 2048, 4096), (2048, 256, 1024),
+    # rows of a decode step whose K is no multiple of 16
+    (3, 40, 100), (4, 4200, 1037),
 ])
 def test_static_linear_equals_quant_then_gemm(native_ops, device, rows, channels, k, xdtype):
     from hif8_rocm import native
@@ -180,6 +182,9 @@ def test_static_linear_equals_quant_then_gemm(native_ops, device, rows, channels
         got = native.static_linear(x, w, scale, ws, b, output_dtype=xdtype)
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        if rows <= 4:
+            fused = native.soft_static_fused_linear(x, w, scale, ws, b, output_dtype=xdtype)
+            assert torch.equal(fused.view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("m", [1, 4])
