@@ -988,6 +988,64 @@ at::Tensor Hif8GatedDelta(const at::Tensor &q, const at::Tensor &k, const at::Te
   return out;
 }
 
+// The causal conv + SiLU of the first conv_weight.size(0) columns of x [B, T, .]
+// (contiguous rows), continued from conv_state [B, C, width - 1]: FP32 [B, T, C].
+at::Tensor Hif8ConvTokens(const at::Tensor &x, const at::Tensor &conv_weight, at::Tensor &conv_state) {
+  CheckContiguousDevice(x, "x");
+  CheckContiguousDevice(conv_weight, "conv_weight");
+  CheckContiguousDevice(conv_state, "conv_state");
+  TORCH_CHECK(x.dim() == 3 && conv_weight.dim() == 2 && conv_state.dim() == 3, "hif8_conv_tokens: operand ranks");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && conv_weight.scalar_type() == at::kBFloat16 &&
+                  conv_state.scalar_type() == at::kBFloat16, "hif8_conv_tokens takes bfloat16 tensors");
+  const int64_t batch = x.size(0), tokens = x.size(1), channels = conv_weight.size(0), width = conv_weight.size(1);
+  TORCH_CHECK(conv_state.size(0) == batch && conv_state.size(1) == channels && conv_state.size(2) == width - 1 &&
+                  x.size(2) >= channels, "hif8_conv_tokens: conv_state [B, C, width - 1], x [B, T, >= C]");
+  CheckSameDevice(conv_weight, x.device(), "conv_weight");
+  CheckSameDevice(conv_state, x.device(), "conv_state");
+  const c10::OptionalDeviceGuard guard(x.device());
+  auto out = at::empty({batch, tokens, channels}, x.options().dtype(at::kFloat));
+  CheckStatus(hif8_conv_tokens(reinterpret_cast<const uint16_t *>(x.data_ptr()), x.size(2),
+                               reinterpret_cast<const uint16_t *>(conv_weight.data_ptr()),
+                               reinterpret_cast<uint16_t *>(conv_state.data_ptr()), out.data_ptr<float>(), batch,
+                               tokens, channels, width, CurrentStream(x.device())),
+              "hif8_conv_tokens");
+  return out;
+}
+
+// bf16(rms_norm(o) * weight * silu(z)): o [B, T, H, dv] FP32 of any strides with
+// contiguous rows, z the columns from z_offset of mixed [B, T, .]; [B, T, H * dv].
+at::Tensor Hif8GatedRmsNorm(const at::Tensor &o, const at::Tensor &mixed, int64_t z_offset, const at::Tensor &weight,
+                            double eps) {
+  CheckContiguousDevice(mixed, "mixed");
+  CheckContiguousDevice(weight, "weight");
+  TORCH_CHECK(o.is_cuda() && o.dim() == 4 && mixed.dim() == 3 && o.scalar_type() == at::kFloat &&
+                  mixed.scalar_type() == at::kBFloat16 && weight.scalar_type() == at::kBFloat16,
+              "hif8_gated_rms_norm: float32 o [B, T, H, dv], bf16 mixed [B, T, .] and weight");
+  const int64_t batch = o.size(0), tokens = o.size(1), heads = o.size(2), dv = o.size(3);
+  TORCH_CHECK(mixed.size(0) == batch && mixed.size(1) == tokens && z_offset >= 0 &&
+                  z_offset + heads * dv <= mixed.size(2) && weight.numel() == dv, "hif8_gated_rms_norm: shapes");
+  CheckSameDevice(mixed, o.device(), "mixed");
+  CheckSameDevice(weight, o.device(), "weight");
+  const c10::OptionalDeviceGuard guard(o.device());
+  const at::Tensor rows = o.stride(3) == 1 ? o : o.contiguous();
+  auto out = at::empty({batch, tokens, heads * dv}, mixed.options());
+  CheckStatus(hif8_gated_rms_norm(rows.data_ptr<float>(), rows.stride(0), rows.stride(1), rows.stride(2),
+                                  reinterpret_cast<const uint16_t *>(mixed.data_ptr()) + z_offset, mixed.size(2),
+                                  reinterpret_cast<const uint16_t *>(weight.data_ptr()),
+                                  reinterpret_cast<uint16_t *>(out.data_ptr()), batch, tokens, heads, dv, float(eps),
+                                  CurrentStream(o.device())),
+              "hif8_gated_rms_norm");
+  return out;
+}
+
+at::Tensor Hif8ConvTokensMeta(const at::Tensor &x, const at::Tensor &conv_weight, at::Tensor &) {
+  return at::empty({x.size(0), x.size(1), conv_weight.size(0)}, x.options().dtype(at::kFloat));
+}
+
+at::Tensor Hif8GatedRmsNormMeta(const at::Tensor &o, const at::Tensor &mixed, int64_t, const at::Tensor &, double) {
+  return at::empty({o.size(0), o.size(1), o.size(2) * o.size(3)}, mixed.options());
+}
+
 at::Tensor Hif8GatedDeltaMeta(const at::Tensor &, const at::Tensor &, const at::Tensor &v, const at::Tensor &,
                               const at::Tensor &, at::Tensor &) {
   return at::empty(v.sizes(), v.options());
@@ -1228,6 +1286,8 @@ TORCH_LIBRARY(vllm_ascend_hif8, m) {
   m.def("hif8_gate_up_silu_mul_quant(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor input_scale) -> (Tensor, Tensor)");
   m.def("hif8_gdn_decode_token(Tensor mixed_qkvz, Tensor x, Tensor ba_weight, Tensor conv_weight, Tensor(a!) conv_state, Tensor a_log, Tensor dt_bias, Tensor(b!) rec_state, Tensor out_norm, int k_heads, int v_heads, int k_dim, int v_dim, float eps) -> Tensor");
   m.def("hif8_linear_conv(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor conv_weight, Tensor(a!) conv_state) -> (Tensor, Tensor)");
+  m.def("hif8_conv_tokens(Tensor x, Tensor conv_weight, Tensor(a!) conv_state) -> Tensor");
+  m.def("hif8_gated_rms_norm(Tensor o, Tensor mixed, int z_offset, Tensor weight, float eps) -> Tensor");
   m.def("hif8_gated_delta(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state) -> Tensor");
   m.def("hif8_gdn_decode_head(Tensor conv, Tensor mixed_qkvz, Tensor x, Tensor ba_weight, Tensor a_log, Tensor dt_bias, Tensor(a!) rec_state, Tensor out_norm, int k_heads, int v_heads, int k_dim, int v_dim, float eps) -> Tensor");
 }
@@ -1255,6 +1315,8 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, CUDA, m) {
   m.impl("hif8_gdn_decode_token", &Hif8GdnDecodeToken);
   m.impl("hif8_gate_up_silu_mul_quant", &Hif8GateUpSiluMulQuant);
   m.impl("hif8_linear_conv", &Hif8LinearConv);
+  m.impl("hif8_conv_tokens", &Hif8ConvTokens);
+  m.impl("hif8_gated_rms_norm", &Hif8GatedRmsNorm);
   m.impl("hif8_gated_delta", &Hif8GatedDelta);
   m.impl("hif8_gdn_decode_head", &Hif8GdnDecodeHead);
   m.impl("soft_hif8_gemm_decoded_weight", &SoftHif8GemmDecodedWeight);
@@ -1286,6 +1348,8 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, Meta, m) {
   m.impl("hif8_gdn_decode_token", &Hif8GdnDecodeTokenMeta);
   m.impl("hif8_gate_up_silu_mul_quant", &Hif8GateUpSiluMulQuantMeta);
   m.impl("hif8_linear_conv", &Hif8LinearConvMeta);
+  m.impl("hif8_conv_tokens", &Hif8ConvTokensMeta);
+  m.impl("hif8_gated_rms_norm", &Hif8GatedRmsNormMeta);
   m.impl("hif8_gated_delta", &Hif8GatedDeltaMeta);
   m.impl("hif8_gdn_decode_head", &Hif8GdnDecodeHeadMeta);
 }

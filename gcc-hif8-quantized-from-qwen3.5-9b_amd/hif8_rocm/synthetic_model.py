@@ -392,12 +392,21 @@ class HybridModel:
         c = self.cfg
         b, t, _ = h.shape
         qkv = L["qkv"](h.reshape(b * t, -1)).reshape(b, t, -1)
-        q, k, v = qkv.split([c.heads * c.head_dim, c.kv_heads * c.head_dim, c.kv_heads * c.head_dim], dim=-1)
-        q = rms_norm(q.reshape(b, t, c.heads, c.head_dim), L["q_norm"], c.rms_eps)
-        k = rms_norm(k.reshape(b, t, c.kv_heads, c.head_dim), L["k_norm"], c.rms_eps)
-        v = v.reshape(b, t, c.kv_heads, c.head_dim)
-        q = self._rope(q, pos)
-        k = self._rope(k, pos)
+        if not decode and c.head_dim <= 256 and b * t <= 65536:
+            # Row i of the fused kernel is one token: norms, rotary and the split
+            # in one launch (its cache slots are not used: _slots below checks them).
+            q, k, v, _ = torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope(
+                qkv.reshape(b * t, -1), L["q_norm"], L["k_norm"], pos.reshape(b * t).to(torch.int64), self.inv_freq,
+                st.block_table[:b].repeat_interleave(t, dim=0), c.block_size, c.heads, c.kv_heads, c.head_dim,
+                c.rms_eps)
+            q, k, v = (x.reshape(b, t, -1, c.head_dim) for x in (q, k, v))
+        else:
+            q, k, v = qkv.split([c.heads * c.head_dim, c.kv_heads * c.head_dim, c.kv_heads * c.head_dim], dim=-1)
+            q = rms_norm(q.reshape(b, t, c.heads, c.head_dim), L["q_norm"], c.rms_eps)
+            k = rms_norm(k.reshape(b, t, c.kv_heads, c.head_dim), L["k_norm"], c.rms_eps)
+            v = v.reshape(b, t, c.kv_heads, c.head_dim)
+            q = self._rope(q, pos)
+            k = self._rope(k, pos)
         if self.calibrating:
             L["k_amax"] = torch.maximum(L["k_amax"], k.float().abs().amax(dim=(0, 1, 3)))
             L["v_amax"] = torch.maximum(L["v_amax"], v.float().abs().amax(dim=(0, 1, 3)))
@@ -434,11 +443,14 @@ class HybridModel:
         gdecay = -torch.exp(L["A_log"]) * torch.nn.functional.softplus(ba[..., c.lin_v_heads:] + L["dt_bias"])
         # Causal depthwise conv over time with the carried state (width conv_kernel).
         conv_state = st.conv_states[idx]
-        seq = torch.cat([conv_state, mixed.transpose(1, 2)], dim=-1)           # [B, C, K-1+T]
-        w = L["conv"].float()
-        acc = sum(seq[..., j: j + t].float() * w[:, j: j + 1] for j in range(c.conv_kernel))
-        conv_state.copy_(seq[..., -(c.conv_kernel - 1):])
-        mixed = torch.nn.functional.silu(acc).transpose(1, 2)                  # [B, T, C]
+        if self._prefill_kernels(t):
+            mixed = torch.ops.vllm_ascend_hif8.hif8_conv_tokens(qkvz, L["conv"], conv_state)
+        else:
+            seq = torch.cat([conv_state, mixed.transpose(1, 2)], dim=-1)       # [B, C, K-1+T]
+            w = L["conv"].float()
+            acc = sum(seq[..., j: j + t].float() * w[:, j: j + 1] for j in range(c.conv_kernel))
+            conv_state.copy_(seq[..., -(c.conv_kernel - 1):])
+            mixed = torch.nn.functional.silu(acc).transpose(1, 2)              # [B, T, C]
         q, k, v = mixed.split([c.lin_qk_width, c.lin_qk_width, c.lin_v_width], dim=-1)
         rep = c.lin_v_heads // c.lin_k_heads
         q = q.reshape(b, t, c.lin_k_heads, c.lin_k_dim).repeat_interleave(rep, dim=2)
@@ -453,10 +465,20 @@ class HybridModel:
             rule = gated_delta_chunked if self.delta_kernel else _gated_delta_torch
             o = rule(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2),
                      gdecay.transpose(1, 2), beta.transpose(1, 2), state).transpose(1, 2)
+        if self._prefill_kernels(t):
+            o = torch.ops.vllm_ascend_hif8.hif8_gated_rms_norm(o, qkvz, 2 * c.lin_qk_width + c.lin_v_width,
+                                                               L["out_norm"], c.rms_eps)
+            return L["out"](o.reshape(b * t, c.lin_v_width)).reshape(b, t, -1)
         zz = z.reshape(b, t, c.lin_v_heads, c.lin_v_dim)
         o = rms_norm(o, L["out_norm"], c.rms_eps).float() * torch.nn.functional.silu(zz.float())
         o = o.to(h.dtype).reshape(b * t, c.lin_v_width)
         return L["out"](o).reshape(b, t, -1)
+
+    def _prefill_kernels(self, t: int) -> bool:
+        """Whether the glue kernels of a prefill take these sizes (t: tokens per request)."""
+        c = self.cfg
+        return (2 <= c.conv_kernel <= 4 and (2 * c.lin_qk_width + c.lin_v_width) % 2 == 0 and c.lin_v_dim % 2 == 0
+                and c.lin_v_dim <= 256 and 0 < t <= 1 << 19)
 
     def _linear_attention_decode(self, L, idx: int, st: RequestState, x: torch.Tensor, xq=None) -> torch.Tensor:
         """One decode token of the linear-attention mixer with the fused glue
@@ -544,11 +566,8 @@ class HybridModel:
         return torch.nn.functional.linear(last, self.lm_head).float()
 
     def _mlp(self, L, h: torch.Tensor) -> torch.Tensor:
-        c = self.cfg
         b, t, _ = h.shape
-        gu = L["gate_up"](h.reshape(b * t, -1))
-        gate, up = gu.split([c.intermediate, c.intermediate], dim=-1)
-        act = (torch.nn.functional.silu(gate.float()) * up.float()).to(h.dtype)
+        act = torch.ops.vllm_ascend_hif8.hif8_silu_mul(L["gate_up"](h.reshape(b * t, -1)))
         return L["down"](act).reshape(b, t, -1)
 
     # -------------------------------------------------------------- forward
@@ -570,18 +589,21 @@ class HybridModel:
         if st.seq_lens is None or not torch.equal(st.seq_lens[:pos.shape[0]].to(torch.int64), want):
             raise ValueError("st.seq_lens must hold each request's length including these tokens "
                              "(the last position + 1) before a prefill forward")
+        add_norm = torch.ops.vllm_ascend_hif8.hif8_add_rms_norm  # h += delta in place; the norm of h
         h = self.embed_method.embedding(self.embed, ids)
+        pending = None
         attn_i = lin_i = 0
         for i, L in enumerate(self.layers):
-            x = rms_norm(h, L["input_norm"], c.rms_eps)
+            x = add_norm(h, pending, L["input_norm"], c.rms_eps)
             if c.is_full_attention(i):
-                h = h + self._attention(L, attn_i, st, x, pos, decode)
+                mix = self._attention(L, attn_i, st, x, pos, decode)
                 attn_i += 1
             else:
-                h = h + self._linear_attention(L, lin_i, st, x, decode)
+                mix = self._linear_attention(L, lin_i, st, x, decode)
                 lin_i += 1
-            h = h + self._mlp(L, rms_norm(h, L["post_norm"], c.rms_eps))
-        last = rms_norm(h[:, -1], self.final_norm, c.rms_eps)
+            pending = self._mlp(L, add_norm(h, mix, L["post_norm"], c.rms_eps))
+        last = add_norm(h[:, -1].contiguous(), None if pending is None else pending[:, -1].contiguous(),
+                        self.final_norm, c.rms_eps)
         return self._lm_head(last)
 
     def calibrate(self, batch: int = 1, tokens: int = 64, seed: int = 1) -> None:

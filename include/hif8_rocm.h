@@ -508,6 +508,22 @@ int hif8_gated_delta(const float *q, const float *k, const float *v, const float
                      int64_t tokens, int64_t k_dim, int64_t v_dim, void *workspace, size_t workspace_bytes,
                      hif8_stream_t stream);
 
+/*
+ * The parts of a linear-attention layer around hif8_gated_delta, over many tokens.
+ * hif8_conv_tokens: out [batch, tokens, channels] FP32 = SiLU of the causal
+ * depthwise conv (width 2..4) over time of the first `channels` columns of x
+ * [batch * tokens, ld] bf16, continued from conv_state [batch, channels,
+ * width - 1] bf16, which is moved on; even channels and ld, 4-byte aligned x.
+ * hif8_gated_rms_norm: out [batch, tokens, heads, v_dim] bf16 = o * rsqrt(mean(o^2)
+ * + eps) * weight * SiLU(z), o FP32 with element strides (batch, token, head) and
+ * contiguous v_dim (even, <= 256), z [batch * tokens, z_ld] bf16.
+ */
+int hif8_conv_tokens(const uint16_t *x, int64_t ld, const uint16_t *conv_weight, uint16_t *conv_state, float *out,
+                     int64_t batch, int64_t tokens, int64_t channels, int64_t conv_width, hif8_stream_t stream);
+int hif8_gated_rms_norm(const float *o, int64_t o_batch, int64_t o_token, int64_t o_head, const uint16_t *z,
+                        int64_t z_ld, const uint16_t *weight, uint16_t *out, int64_t batch, int64_t tokens,
+                        int64_t heads, int64_t v_dim, float eps, hif8_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -62,3 +62,43 @@ def test_gated_delta_leaves_autograd_and_other_types_to_torch(native_ops, device
     assert not takes(*tensors[:2], tensors[2].requires_grad_(), *tensors[3:], state, 64)
     with torch.no_grad():
         assert takes(*tensors, state, 64)
+
+
+@pytest.mark.parametrize("b,t,channels,width,ld", [(1, 1, 64, 4, 80), (2, 2, 64, 3, 70), (3, 3, 66, 4, 66),
+                                                   (2, 16, 514, 2, 520), (1, 49, 1026, 4, 1030)])
+def test_conv_tokens_equals_the_elementwise_form(native_ops, device, b, t, channels, width, ld):
+    """Bit for bit, with fewer tokens than the state is long, run edges and a padded row pitch."""
+    g = torch.Generator().manual_seed(t + channels)
+    x = torch.randn(b, t, ld, generator=g).to(torch.bfloat16).to(device)
+    w = torch.randn(channels, width, generator=g).to(torch.bfloat16).to(device)
+    state = torch.randn(b, channels, width - 1, generator=g).to(torch.bfloat16).to(device)
+    seq = torch.cat([state, x[..., :channels].transpose(1, 2)], dim=-1)
+    acc = sum(seq[..., j:j + t].float() * w.float()[:, j:j + 1] for j in range(width))
+    got = torch.ops.vllm_ascend_hif8.hif8_conv_tokens(x, w, state)
+    torch.cuda.synchronize()
+    assert torch.equal(got, torch.nn.functional.silu(acc).transpose(1, 2))
+    assert torch.equal(state, seq[..., -(width - 1):])
+
+
+@pytest.mark.parametrize("b,t,h,dv,offset", [(1, 1, 1, 2, 0), (2, 5, 3, 128, 6), (1, 4, 2, 130, 2), (1, 3, 2, 256, 0)])
+def test_gated_rms_norm_matches_torch(native_ops, device, b, t, h, dv, offset):
+    g = torch.Generator().manual_seed(dv + h)
+    o = torch.randn(b, h, t, dv, generator=g).to(device).transpose(1, 2)
+    mixed = torch.randn(b, t, offset + h * dv + 2, generator=g).to(torch.bfloat16).to(device)
+    w = torch.randn(dv, generator=g).to(torch.bfloat16).to(device)
+    z = mixed[..., offset:offset + h * dv].reshape(b, t, h, dv).double()
+    want = synthetic_model.rms_norm(o, w, 1e-6).double() * torch.nn.functional.silu(z)
+    got = torch.ops.vllm_ascend_hif8.hif8_gated_rms_norm(o, mixed, offset, w, 1e-6)
+    torch.cuda.synchronize()
+    # One rounding to bf16: eight significant bits, so at most 2^-8 of the value
+    # (ulp 2^-7 at 1, half of it), plus FP32 terms of ~1e-6.
+    torch.testing.assert_close(got.double(), want.reshape(b, t, -1), rtol=2 ** -8 + 1e-5, atol=1e-30)
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 24), (5, 6), (300, 1024)])
+def test_silu_mul_equals_torch(native_ops, device, rows, n):
+    g = torch.Generator().manual_seed(n)
+    gu = (torch.randn(rows, 2 * n, generator=g) * 4).to(torch.bfloat16).to(device)
+    gate, up = gu.float().split([n, n], dim=-1)
+    assert torch.equal(torch.ops.vllm_ascend_hif8.hif8_silu_mul(gu),
+                       (torch.nn.functional.silu(gate) * up).to(torch.bfloat16))
