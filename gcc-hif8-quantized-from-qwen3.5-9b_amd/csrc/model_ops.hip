@@ -42,6 +42,13 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
   return s;
 }
 
+// The static HiF8 code of one bf16 value with fixed scale s, as
+// hif8_static_quant encodes it, by division and the format rules (for a kernel
+// with one value per thread the table's copy into LDS would cost more).
+__device__ __forceinline__ uint8_t static_code(float v, float s) {
+  return uint8_t(static_encode_bits(__float_as_uint(v / s)));
+}
+
 constexpr int kNormThreads = 256;
 
 template <bool kResidual>
@@ -646,12 +653,17 @@ __global__ __launch_bounds__(kGdnWideThreads) void gdn_token_kernel(
 // b = 1 (16 key heads, 32 value heads, dk = dv = 128) 6.8 us per call in the
 // decode step's kernel trace against 12.5 us for the group kernel.  Requires
 // dk = 8 kR, dv <= 128, hidden % 8 == 0, hidden <= 8192.
-template <int kR>
+// kQuant: instead of the bf16 row, its static HiF8 codes with the fixed scale
+// qs[0] (the out projection's input quant) and row_scale[b] = qs[0]: each lead
+// thread encodes its one value, which saves the quant launch (5 us of a decode
+// step's linear-attention layer on MI355X).
+template <int kR, bool kQuant>
 __global__ __launch_bounds__(kGdnWideThreads) void gdn_head_kernel(
     const float *__restrict__ conv, const uint16_t *__restrict__ mixed, int64_t ld, const uint16_t *__restrict__ x,
     const uint16_t *__restrict__ w_ba, int hidden, const float *__restrict__ a_log,
     const float *__restrict__ dt_bias, float *__restrict__ state, const uint16_t *__restrict__ w_out,
-    uint16_t *__restrict__ out, int k_heads, int v_heads, int dv, float eps) {
+    uint16_t *__restrict__ out, int k_heads, int v_heads, int dv, float eps, const float *__restrict__ qs_in,
+    uint8_t *__restrict__ codes, float *__restrict__ row_scale) {
   constexpr int dk = kGdnParts * kR;
   __shared__ __attribute__((aligned(16))) float qs[dk], ks[dk];  // raw conv outputs of q and k
   __shared__ float pa[kGdnParts][kGdnCols], pc[kGdnParts][kGdnCols];
@@ -764,8 +776,12 @@ __global__ __launch_bounds__(kGdnWideThreads) void gdn_head_kernel(
   if (part == 0 && col_ok) {
     const float rn = rsqrtf((o_red[0] + o_red[1]) / float(dv) + eps);
     const float z = bf(uint16_t(zraw));
-    out[(size_t(b) * v_heads + hv) * dv + j] = to_bf(o * rn * bf(uint16_t(wo)) * (z / (1.f + expf(-z))));
+    const uint16_t y = to_bf(o * rn * bf(uint16_t(wo)) * (z / (1.f + expf(-z))));
+    const size_t at = (size_t(b) * v_heads + hv) * dv + j;
+    if constexpr (kQuant) codes[at] = static_code(bf(y), qs_in[0]);
+    else out[at] = y;
   }
+  if (kQuant && hv == 0 && tid == 0) row_scale[b] = qs_in[0];
 }
 
 constexpr int kHeadThreads = 256;
@@ -774,11 +790,22 @@ constexpr int kHeadThreads = 256;
 // RMS-normalised (weight w_q / w_k) and rotated on their first rot dims
 // (halves i, i + rot/2, angle pos * inv_freq[i]); v heads copied.  Block
 // (b, 0) also writes the cache slot of position pos[b].
+// kCache: k and v heads go to that slot of the paged cache instead, as
+// hif8_kv_cache_write would put them there: static HiF8 codes with the head's
+// scale, then the scale itself (one value per thread; a launch less per layer).
+struct CacheRows {
+  uint8_t *key = nullptr, *value = nullptr;  // [num_blocks, block_size, hkv, d + 4]
+  const float *key_scale = nullptr, *value_scale = nullptr;  // [hkv]
+  int64_t num_blocks = 0;
+};
+
+template <bool kCache>
 __global__ __launch_bounds__(kHeadThreads) void qk_norm_rope_kernel(
     const uint16_t *__restrict__ qkv, const uint16_t *__restrict__ w_q, const uint16_t *__restrict__ w_k,
     const int64_t *__restrict__ pos, const float *__restrict__ inv_freq, const int32_t *__restrict__ block_table,
     int64_t max_blocks, int block_size, uint16_t *__restrict__ q_out, uint16_t *__restrict__ k_out,
-    uint16_t *__restrict__ v_out, int64_t *__restrict__ slots, int hq, int hkv, int d, int rot, float eps) {
+    uint16_t *__restrict__ v_out, int64_t *__restrict__ slots, int hq, int hkv, int d, int rot, float eps,
+    const CacheRows cache) {
   __shared__ float y[kHeadThreads];
   __shared__ float red[kHeadThreads / kWave];
   const int heads = hq + 2 * hkv;
@@ -797,8 +824,29 @@ __global__ __launch_bounds__(kHeadThreads) void qk_norm_rope_kernel(
     }
     slots[b] = slot;
   }
+  // The cache row of this block's k or v head; null past the table or the cache.
+  uint8_t *row = nullptr;
+  float scale = 1.f;
+  if constexpr (kCache) {
+    if (h >= hq && p >= 0 && p / block_size < max_blocks) {
+      const bool is_v = h >= hq + hkv;
+      const int kv = h - hq - (is_v ? hkv : 0);
+      const int64_t blk = block_table[size_t(b) * max_blocks + p / block_size];
+      if (blk >= 0 && blk < cache.num_blocks) {
+        row = (is_v ? cache.value : cache.key) + ((blk * block_size + p % block_size) * hkv + kv) * (d + 4);
+        scale = (is_v ? cache.value_scale : cache.key_scale)[kv];
+        if (j == 0) *reinterpret_cast<float *>(row + d) = scale;
+      }
+    }
+  }
   if (h >= hq + hkv) {
-    if (j < d) v_out[(size_t(b) * hkv + (h - hq - hkv)) * d + j] = qkv[(size_t(b) * heads + h) * d + j];
+    if (j < d) {
+      if constexpr (kCache) {
+        if (row) row[j] = static_code(x, scale);
+      } else {
+        v_out[(size_t(b) * hkv + (h - hq - hkv)) * d + j] = qkv[(size_t(b) * heads + h) * d + j];
+      }
+    }
     return;
   }
   const bool is_q = h < hq;
@@ -814,8 +862,12 @@ __global__ __launch_bounds__(kHeadThreads) void qk_norm_rope_kernel(
     out = j < half ? y[j] * c - y[j + half] * s : y[j] * c + y[j - half] * s;
   }
   if (j < d) {
-    uint16_t *dst = is_q ? q_out + (size_t(b) * hq + h) * d : k_out + (size_t(b) * hkv + (h - hq)) * d;
-    dst[j] = to_bf(out);
+    if (kCache && !is_q) {
+      if (row) row[j] = static_code(bf(to_bf(out)), scale);
+    } else {
+      uint16_t *dst = is_q ? q_out + (size_t(b) * hq + h) * d : k_out + (size_t(b) * hkv + (h - hq)) * d;
+      dst[j] = to_bf(out);
+    }
   }
 }
 
@@ -836,11 +888,40 @@ extern "C" int hif8_qk_norm_rope(const uint16_t *qkv, const uint16_t *q_norm, co
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||
       rotary_dim < 0 || rotary_dim > head_size || rotary_dim % 2 || block_size <= 0 || batch > 65536)
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope: unsupported dimensions");
-  qk_norm_rope_kernel<<<unsigned(batch * (num_heads + 2 * num_kv_heads)), kHeadThreads, 0,
-                        reinterpret_cast<hipStream_t>(stream)>>>(
+  qk_norm_rope_kernel<false><<<unsigned(batch * (num_heads + 2 * num_kv_heads)), kHeadThreads, 0,
+                               reinterpret_cast<hipStream_t>(stream)>>>(
       qkv, q_norm, k_norm, pos, inv_freq, block_table, max_blocks, int(block_size), q_out, k_out, v_out, slots,
-      int(num_heads), int(num_kv_heads), int(head_size), int(rotary_dim), eps);
+      int(num_heads), int(num_kv_heads), int(head_size), int(rotary_dim), eps, CacheRows());
   return check_launch("hif8_qk_norm_rope");
+}
+
+extern "C" int hif8_qk_norm_rope_cache(const uint16_t *qkv, const uint16_t *q_norm, const uint16_t *k_norm,
+                                       const int64_t *pos, const float *inv_freq, const int32_t *block_table,
+                                       int64_t max_blocks, int64_t num_blocks, int64_t block_size, uint16_t *q_out,
+                                       uint8_t *key_cache, uint8_t *value_cache, const float *key_scale,
+                                       const float *value_scale, int64_t batch, int64_t num_heads,
+                                       int64_t num_kv_heads, int64_t head_size, int64_t rotary_dim, float eps,
+                                       hif8_stream_t stream) {
+  clear_error();
+  if (!qkv || !q_norm || !k_norm || !pos || !inv_freq || !block_table || !q_out || !key_cache || !value_cache ||
+      !key_scale || !value_scale)
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope_cache: null pointer argument");
+  if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||
+      head_size % 4 || rotary_dim < 0 || rotary_dim > head_size || rotary_dim % 2 || block_size <= 0 ||
+      block_size > 0x7FFFFFFFll || num_blocks <= 0 || batch > 65536 || !aligned(key_cache, 4) ||
+      !aligned(value_cache, 4))
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope_cache: unsupported dimensions");
+  CacheRows cache;
+  cache.key = key_cache;
+  cache.value = value_cache;
+  cache.key_scale = key_scale;
+  cache.value_scale = value_scale;
+  cache.num_blocks = num_blocks;
+  qk_norm_rope_kernel<true><<<unsigned(batch * (num_heads + 2 * num_kv_heads)), kHeadThreads, 0,
+                              reinterpret_cast<hipStream_t>(stream)>>>(
+      qkv, q_norm, k_norm, pos, inv_freq, block_table, max_blocks, int(block_size), q_out, nullptr, nullptr, nullptr,
+      int(num_heads), int(num_kv_heads), int(head_size), int(rotary_dim), eps, cache);
+  return check_launch("hif8_qk_norm_rope_cache");
 }
 
 extern "C" int hif8_add_rms_norm(uint16_t *h, const uint16_t *delta, const uint16_t *weight, uint16_t *out,
@@ -987,37 +1068,66 @@ extern "C" int hif8_gdn_decode_token(const uint16_t *mixed_qkvz, int64_t ld, con
   return check_launch("hif8_gdn_decode_token");
 }
 
+namespace {
+
+// hif8_gdn_decode_head, or with codes set hif8_gdn_decode_head_quant (out unused).
+int launch_gdn_head(const char *op, const float *conv, const uint16_t *mixed_qkvz, int64_t ld, const uint16_t *x,
+                    const uint16_t *ba_weight, int64_t hidden, const float *a_log, const float *dt_bias,
+                    float *rec_state, const uint16_t *out_norm, uint16_t *out, const float *input_scale,
+                    uint8_t *codes, float *row_scale, int64_t batch, int64_t k_heads, int64_t v_heads, int64_t k_dim,
+                    int64_t v_dim, float eps, hif8_stream_t stream) {
+  clear_error();
+  if (!conv || !mixed_qkvz || !x || !ba_weight || !a_log || !dt_bias || !rec_state || !out_norm ||
+      !(out || (input_scale && codes && row_scale)))
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "%s: null pointer argument", op);
+  if (batch <= 0 || k_heads <= 0 || v_heads <= 0 || v_heads % k_heads || k_dim <= 0 || v_dim <= 0 ||
+      hidden <= 0 || hidden > 0x7FFFFFFFll || batch * v_heads > 0x7FFFFFFFll)
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "%s: unsupported dimensions", op);
+  const int64_t channels = 2 * k_heads * k_dim + v_heads * v_dim;
+  if (ld < channels + v_heads * v_dim)
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "%s: mixed_qkvz row too short", op);
+  const int64_t rows = k_dim / kGdnParts;
+  if (k_dim % kGdnParts || (rows != 16 && rows != 8 && rows != 4) || v_dim > kGdnCols || hidden % 8 ||
+      hidden > 8 * kNormThreads * 4 || !aligned(x, 16) || !aligned(ba_weight, 16))
+    return fail(HIF8_ERR_UNSUPPORTED, "%s: needs k_dim in {32, 64, 128}, v_dim <= 128, "
+                                      "hidden %% 8 == 0, hidden <= 8192 and 16-byte aligned x / ba_weight", op);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const dim3 grid(unsigned(batch * v_heads));
+  auto go = [&](auto kern) {
+    kern<<<grid, kGdnWideThreads, 0, s>>>(conv, mixed_qkvz, ld, x, ba_weight, int(hidden), a_log, dt_bias, rec_state,
+                                          out_norm, out, int(k_heads), int(v_heads), int(v_dim), eps, input_scale,
+                                          codes, row_scale);
+  };
+  if (rows == 16) codes ? go(gdn_head_kernel<16, true>) : go(gdn_head_kernel<16, false>);
+  else if (rows == 8) codes ? go(gdn_head_kernel<8, true>) : go(gdn_head_kernel<8, false>);
+  else codes ? go(gdn_head_kernel<4, true>) : go(gdn_head_kernel<4, false>);
+  return check_launch(op);
+}
+
+}  // namespace
+
 extern "C" int hif8_gdn_decode_head(const float *conv, const uint16_t *mixed_qkvz, int64_t ld, const uint16_t *x,
                                     const uint16_t *ba_weight, int64_t hidden, const float *a_log,
                                     const float *dt_bias, float *rec_state, const uint16_t *out_norm, uint16_t *out,
                                     int64_t batch, int64_t k_heads, int64_t v_heads, int64_t k_dim, int64_t v_dim,
                                     float eps, hif8_stream_t stream) {
-  clear_error();
-  if (!conv || !mixed_qkvz || !x || !ba_weight || !a_log || !dt_bias || !rec_state || !out_norm || !out)
-    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_gdn_decode_head: null pointer argument");
-  if (batch <= 0 || k_heads <= 0 || v_heads <= 0 || v_heads % k_heads || k_dim <= 0 || v_dim <= 0 ||
-      hidden <= 0 || hidden > 0x7FFFFFFFll || batch * v_heads > 0x7FFFFFFFll)
-    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_gdn_decode_head: unsupported dimensions");
-  const int64_t channels = 2 * k_heads * k_dim + v_heads * v_dim;
-  if (ld < channels + v_heads * v_dim)
-    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_gdn_decode_head: mixed_qkvz row too short");
-  const int64_t rows = k_dim / kGdnParts;
-  if (k_dim % kGdnParts || (rows != 16 && rows != 8 && rows != 4) || v_dim > kGdnCols || hidden % 8 ||
-      hidden > 8 * kNormThreads * 4 || !aligned(x, 16) || !aligned(ba_weight, 16))
-    return fail(HIF8_ERR_UNSUPPORTED, "hif8_gdn_decode_head: needs k_dim in {32, 64, 128}, v_dim <= 128, "
-                                      "hidden %% 8 == 0, hidden <= 8192 and 16-byte aligned x / ba_weight");
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(unsigned(batch * v_heads));
-#define HIF8_GDN_HEAD(R)                                                                                    \
-  gdn_head_kernel<R><<<grid, kGdnWideThreads, 0, s>>>(conv, mixed_qkvz, ld, x, ba_weight, int(hidden), a_log, \
-                                                      dt_bias, rec_state, out_norm, out, int(k_heads),        \
-                                                      int(v_heads), int(v_dim), eps)
-  if (rows == 16) HIF8_GDN_HEAD(16);
-  else if (rows == 8) HIF8_GDN_HEAD(8);
-  else HIF8_GDN_HEAD(4);
-#undef HIF8_GDN_HEAD
-  return check_launch("hif8_gdn_decode_head");
+  return launch_gdn_head("hif8_gdn_decode_head", conv, mixed_qkvz, ld, x, ba_weight, hidden, a_log, dt_bias, rec_state,
+                         out_norm, out, nullptr, nullptr, nullptr, batch, k_heads, v_heads, k_dim, v_dim, eps, stream);
 }
+
+extern "C" int hif8_gdn_decode_head_quant(const float *conv, const uint16_t *mixed_qkvz, int64_t ld, const uint16_t *x,
+                                          const uint16_t *ba_weight, int64_t hidden, const float *a_log,
+                                          const float *dt_bias, float *rec_state, const uint16_t *out_norm,
+                                          const float *input_scale, uint8_t *codes, float *row_scale, int64_t batch,
+                                          int64_t k_heads, int64_t v_heads, int64_t k_dim, int64_t v_dim, float eps,
+                                          hif8_stream_t stream) {
+  if (!input_scale || !codes || !row_scale)
+    return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_gdn_decode_head_quant: null pointer argument");
+  return launch_gdn_head("hif8_gdn_decode_head_quant", conv, mixed_qkvz, ld, x, ba_weight, hidden, a_log, dt_bias,
+                         rec_state, out_norm, nullptr, input_scale, codes, row_scale, batch, k_heads, v_heads, k_dim,
+                         v_dim, eps, stream);
+}
+
 
 extern "C" int hif8_gdn_decode_step(const uint16_t *mixed_qkvz, int64_t ld, const uint16_t *ba,
                                     const uint16_t *conv_weight, uint16_t *conv_state, const float *a_log,

@@ -907,10 +907,10 @@ at::Tensor Hif8GdnDecodeStep(const at::Tensor &mixed, const at::Tensor &ba, cons
 
 // The recurrence of one decode token from hif8_linear_conv's conv outputs,
 // the b/a projection of x folded in, one block per (request, value head).
-at::Tensor Hif8GdnDecodeHead(const at::Tensor &conv, const at::Tensor &mixed, const at::Tensor &x,
-                             const at::Tensor &ba_weight, const at::Tensor &a_log, const at::Tensor &dt_bias,
-                             at::Tensor &rec_state, const at::Tensor &out_norm, int64_t k_heads, int64_t v_heads,
-                             int64_t k_dim, int64_t v_dim, double eps) {
+void CheckGdnDecodeHead(const at::Tensor &conv, const at::Tensor &mixed, const at::Tensor &x,
+                        const at::Tensor &ba_weight, const at::Tensor &a_log, const at::Tensor &dt_bias,
+                        const at::Tensor &rec_state, const at::Tensor &out_norm, int64_t k_heads, int64_t v_heads,
+                        int64_t k_dim, int64_t v_dim) {
   for (auto *t : {&conv, &mixed, &x, &ba_weight, &a_log, &dt_bias, &out_norm}) CheckContiguousDevice(*t, "operand");
   CheckContiguousDevice(rec_state, "rec_state");
   TORCH_CHECK(conv.dim() == 2 && mixed.dim() == 2 && x.dim() == 2 && ba_weight.dim() == 2 && rec_state.dim() == 4,
@@ -931,6 +931,14 @@ at::Tensor Hif8GdnDecodeHead(const at::Tensor &conv, const at::Tensor &mixed, co
                   rec_state.size(3) == v_dim, "rec_state must be [batch, v_heads, k_dim, v_dim]");
   TORCH_CHECK(a_log.numel() == v_heads && dt_bias.numel() == v_heads && out_norm.numel() == v_dim,
               "per-head parameters");
+}
+
+at::Tensor Hif8GdnDecodeHead(const at::Tensor &conv, const at::Tensor &mixed, const at::Tensor &x,
+                             const at::Tensor &ba_weight, const at::Tensor &a_log, const at::Tensor &dt_bias,
+                             at::Tensor &rec_state, const at::Tensor &out_norm, int64_t k_heads, int64_t v_heads,
+                             int64_t k_dim, int64_t v_dim, double eps) {
+  CheckGdnDecodeHead(conv, mixed, x, ba_weight, a_log, dt_bias, rec_state, out_norm, k_heads, v_heads, k_dim, v_dim);
+  const int64_t batch = conv.size(0);
   const c10::OptionalDeviceGuard guard(conv.device());
   auto out = at::empty({batch, v_heads * v_dim}, mixed.options());
   CheckStatus(hif8_gdn_decode_head(conv.data_ptr<float>(), reinterpret_cast<const uint16_t *>(mixed.data_ptr()),
@@ -942,6 +950,39 @@ at::Tensor Hif8GdnDecodeHead(const at::Tensor &conv, const at::Tensor &mixed, co
                                    v_dim, float(eps), CurrentStream(conv.device())),
               "hif8_gdn_decode_head");
   return out;
+}
+
+// Hif8GdnDecodeHead with its output as the out projection's static codes.
+std::tuple<at::Tensor, at::Tensor> Hif8GdnDecodeHeadQuant(
+    const at::Tensor &conv, const at::Tensor &mixed, const at::Tensor &x, const at::Tensor &ba_weight,
+    const at::Tensor &a_log, const at::Tensor &dt_bias, at::Tensor &rec_state, const at::Tensor &out_norm,
+    const at::Tensor &input_scale, int64_t k_heads, int64_t v_heads, int64_t k_dim, int64_t v_dim, double eps) {
+  CheckGdnDecodeHead(conv, mixed, x, ba_weight, a_log, dt_bias, rec_state, out_norm, k_heads, v_heads, k_dim, v_dim);
+  CheckContiguousDevice(input_scale, "input_scale");
+  TORCH_CHECK(input_scale.scalar_type() == at::kFloat && input_scale.numel() == 1,
+              "hif8_gdn_decode_head_quant: one float32 input scale");
+  const int64_t batch = conv.size(0);
+  const c10::OptionalDeviceGuard guard(conv.device());
+  auto codes = at::empty({batch, v_heads * v_dim}, mixed.options().dtype(at::kByte));
+  auto row_scale = at::empty({batch}, mixed.options().dtype(at::kFloat));
+  CheckStatus(hif8_gdn_decode_head_quant(
+                  conv.data_ptr<float>(), reinterpret_cast<const uint16_t *>(mixed.data_ptr()), mixed.size(1),
+                  reinterpret_cast<const uint16_t *>(x.data_ptr()),
+                  reinterpret_cast<const uint16_t *>(ba_weight.data_ptr()), x.size(1), a_log.data_ptr<float>(),
+                  dt_bias.data_ptr<float>(), rec_state.data_ptr<float>(),
+                  reinterpret_cast<const uint16_t *>(out_norm.data_ptr()), input_scale.data_ptr<float>(),
+                  codes.data_ptr<uint8_t>(), row_scale.data_ptr<float>(), batch, k_heads, v_heads, k_dim, v_dim,
+                  float(eps), CurrentStream(conv.device())),
+              "hif8_gdn_decode_head_quant");
+  return {codes, row_scale};
+}
+
+std::tuple<at::Tensor, at::Tensor> Hif8GdnDecodeHeadQuantMeta(
+    const at::Tensor &conv, const at::Tensor &mixed, const at::Tensor &, const at::Tensor &, const at::Tensor &,
+    const at::Tensor &, at::Tensor &, const at::Tensor &, const at::Tensor &, int64_t, int64_t v_heads, int64_t,
+    int64_t v_dim, double) {
+  return {at::empty({conv.size(0), v_heads * v_dim}, mixed.options().dtype(at::kByte)),
+          at::empty({conv.size(0)}, mixed.options().dtype(at::kFloat))};
 }
 
 // The gated delta rule over many tokens: q, k [B, H, T, dk], v [B, H, T, dv], g,
@@ -1132,6 +1173,48 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> Hif8QkNormRope(
 
 // ------------------------------------------------------------------ Meta
 
+// hif8_qk_norm_rope and the cache write of its k and v in one launch; returns q.
+at::Tensor Hif8QkNormRopeCache(const at::Tensor &qkv, const at::Tensor &q_norm, const at::Tensor &k_norm,
+                               const at::Tensor &pos, const at::Tensor &inv_freq, const at::Tensor &block_table,
+                               at::Tensor &key_cache, at::Tensor &value_cache, const at::Tensor &key_scale,
+                               const at::Tensor &value_scale, int64_t num_heads, double eps) {
+  for (auto *t : {&qkv, &q_norm, &k_norm, &pos, &inv_freq, &block_table, &key_scale, &value_scale})
+    CheckContiguousDevice(*t, "operand");
+  CheckContiguousDevice(key_cache, "key_cache");
+  CheckContiguousDevice(value_cache, "value_cache");
+  TORCH_CHECK(qkv.scalar_type() == at::kBFloat16 && q_norm.scalar_type() == at::kBFloat16 &&
+                  k_norm.scalar_type() == at::kBFloat16, "hif8_qk_norm_rope_cache: bf16 qkv and norms");
+  TORCH_CHECK(pos.scalar_type() == at::kLong && inv_freq.scalar_type() == at::kFloat &&
+                  block_table.scalar_type() == at::kInt && key_scale.scalar_type() == at::kFloat &&
+                  value_scale.scalar_type() == at::kFloat,
+              "hif8_qk_norm_rope_cache: int64 pos, float32 inv_freq and scales, int32 table");
+  TORCH_CHECK(key_cache.scalar_type() == at::kByte && key_cache.dim() == 4 && value_cache.scalar_type() == at::kByte &&
+                  value_cache.sizes() == key_cache.sizes(), "hif8_qk_norm_rope_cache: uint8 caches of one shape");
+  const int64_t batch = qkv.size(0), kv_heads = key_cache.size(2), head_size = key_cache.size(3) - 4;
+  TORCH_CHECK(head_size > 0 && qkv.numel() == batch * (num_heads + 2 * kv_heads) * head_size, "qkv width");
+  TORCH_CHECK(q_norm.numel() == head_size && k_norm.numel() == head_size && key_scale.numel() == kv_heads &&
+                  value_scale.numel() == kv_heads, "norm weights and scales");
+  TORCH_CHECK(pos.numel() == batch && block_table.dim() == 2 && block_table.size(0) >= batch, "pos / block_table");
+  const c10::OptionalDeviceGuard guard(qkv.device());
+  auto q = at::empty({batch, num_heads, head_size}, qkv.options());
+  CheckStatus(hif8_qk_norm_rope_cache(
+                  reinterpret_cast<const uint16_t *>(qkv.data_ptr()),
+                  reinterpret_cast<const uint16_t *>(q_norm.data_ptr()),
+                  reinterpret_cast<const uint16_t *>(k_norm.data_ptr()), pos.data_ptr<int64_t>(),
+                  inv_freq.data_ptr<float>(), block_table.data_ptr<int32_t>(), block_table.size(1), key_cache.size(0),
+                  key_cache.size(1), reinterpret_cast<uint16_t *>(q.data_ptr()), key_cache.data_ptr<uint8_t>(),
+                  value_cache.data_ptr<uint8_t>(), key_scale.data_ptr<float>(), value_scale.data_ptr<float>(), batch,
+                  num_heads, kv_heads, head_size, 2 * inv_freq.numel(), float(eps), CurrentStream(qkv.device())),
+              "hif8_qk_norm_rope_cache");
+  return q;
+}
+
+at::Tensor Hif8QkNormRopeCacheMeta(const at::Tensor &qkv, const at::Tensor &, const at::Tensor &, const at::Tensor &,
+                                   const at::Tensor &, const at::Tensor &, at::Tensor &key_cache, at::Tensor &,
+                                   const at::Tensor &, const at::Tensor &, int64_t num_heads, double) {
+  return at::empty({qkv.size(0), num_heads, key_cache.size(3) - 4}, qkv.options());
+}
+
 std::tuple<at::Tensor, at::Tensor> Hif8StaticQuantMeta(const at::Tensor &x, const at::Tensor &fixed_scale) {
   (void)fixed_scale;
   auto data = at::empty_like(x, x.options().dtype(at::kByte));
@@ -1286,6 +1369,8 @@ TORCH_LIBRARY(vllm_ascend_hif8, m) {
   m.def("hif8_gate_up_silu_mul_quant(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor input_scale) -> (Tensor, Tensor)");
   m.def("hif8_gdn_decode_token(Tensor mixed_qkvz, Tensor x, Tensor ba_weight, Tensor conv_weight, Tensor(a!) conv_state, Tensor a_log, Tensor dt_bias, Tensor(b!) rec_state, Tensor out_norm, int k_heads, int v_heads, int k_dim, int v_dim, float eps) -> Tensor");
   m.def("hif8_linear_conv(Tensor activation, Tensor weight, Tensor token_scale, Tensor channel_scale, Tensor conv_weight, Tensor(a!) conv_state) -> (Tensor, Tensor)");
+  m.def("hif8_gdn_decode_head_quant(Tensor conv, Tensor mixed_qkvz, Tensor x, Tensor ba_weight, Tensor a_log, Tensor dt_bias, Tensor(a!) rec_state, Tensor out_norm, Tensor input_scale, int k_heads, int v_heads, int k_dim, int v_dim, float eps) -> (Tensor, Tensor)");
+  m.def("hif8_qk_norm_rope_cache(Tensor qkv, Tensor q_norm, Tensor k_norm, Tensor pos, Tensor inv_freq, Tensor block_table, Tensor(a!) key_cache, Tensor(b!) value_cache, Tensor key_scale, Tensor value_scale, int num_heads, float eps) -> Tensor");
   m.def("hif8_conv_tokens(Tensor x, Tensor conv_weight, Tensor(a!) conv_state) -> Tensor");
   m.def("hif8_gated_rms_norm(Tensor o, Tensor mixed, int z_offset, Tensor weight, float eps) -> Tensor");
   m.def("hif8_gated_delta(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state) -> Tensor");
@@ -1315,6 +1400,8 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, CUDA, m) {
   m.impl("hif8_gdn_decode_token", &Hif8GdnDecodeToken);
   m.impl("hif8_gate_up_silu_mul_quant", &Hif8GateUpSiluMulQuant);
   m.impl("hif8_linear_conv", &Hif8LinearConv);
+  m.impl("hif8_gdn_decode_head_quant", &Hif8GdnDecodeHeadQuant);
+  m.impl("hif8_qk_norm_rope_cache", &Hif8QkNormRopeCache);
   m.impl("hif8_conv_tokens", &Hif8ConvTokens);
   m.impl("hif8_gated_rms_norm", &Hif8GatedRmsNorm);
   m.impl("hif8_gated_delta", &Hif8GatedDelta);
@@ -1348,6 +1435,8 @@ TORCH_LIBRARY_IMPL(vllm_ascend_hif8, Meta, m) {
   m.impl("hif8_gdn_decode_token", &Hif8GdnDecodeTokenMeta);
   m.impl("hif8_gate_up_silu_mul_quant", &Hif8GateUpSiluMulQuantMeta);
   m.impl("hif8_linear_conv", &Hif8LinearConvMeta);
+  m.impl("hif8_gdn_decode_head_quant", &Hif8GdnDecodeHeadQuantMeta);
+  m.impl("hif8_qk_norm_rope_cache", &Hif8QkNormRopeCacheMeta);
   m.impl("hif8_conv_tokens", &Hif8ConvTokensMeta);
   m.impl("hif8_gated_rms_norm", &Hif8GatedRmsNormMeta);
   m.impl("hif8_gated_delta", &Hif8GatedDeltaMeta);

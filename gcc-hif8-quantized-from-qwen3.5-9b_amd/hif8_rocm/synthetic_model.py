@@ -379,6 +379,15 @@ class HybridModel:
         c = self.cfg
         b = x.shape[0]
         qkv = L["qkv"](x) if xq is None else L["qkv"].from_codes(*xq)
+        if xq is not None and c.head_dim % 4 == 0 and c.head_dim <= 256:
+            # Norms, rotary and the cache write of k and v in one launch.
+            q = torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope_cache(
+                qkv, L["q_norm"], L["k_norm"], pos.reshape(b), self.inv_freq, st.block_table, st.key_caches[idx],
+                st.value_caches[idx], L["k_scale"], L["v_scale"], c.heads, c.rms_eps)
+            o = kv_cache.paged_decode_attention(q, st.key_caches[idx], st.value_caches[idx], st.block_table,
+                                                st.seq_lens, scale=1.0 / math.sqrt(c.head_dim),
+                                                max_seq_len=st.max_len, validate=False)
+            return L["o"](o.reshape(b, c.heads * c.head_dim))
         q, k, v, slots = torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope(
             qkv, L["q_norm"], L["k_norm"], pos.reshape(b), self.inv_freq, st.block_table, c.block_size, c.heads,
             c.kv_heads, c.head_dim, c.rms_eps)
@@ -489,12 +498,13 @@ class HybridModel:
         ops = torch.ops.vllm_ascend_hif8
         if xq is not None and self._head_split_ok(x.shape[0]):
             # Two launches: the qkvz GEMV with the conv in its epilogue, then
-            # one block per (request, value head) for the recurrence.
+            # one block per (request, value head) for the recurrence, which
+            # also quantizes the out projection's input.
             qkvz, conv = L["qkvz"].conv_from_codes(*xq, L["conv"], st.conv_states[idx])
-            o = ops.hif8_gdn_decode_head(conv, qkvz, x, L["ba"], L["A_log"], L["dt_bias"], st.rec_states[idx],
-                                         L["out_norm"], c.lin_k_heads, c.lin_v_heads, c.lin_k_dim, c.lin_v_dim,
-                                         c.rms_eps)
-            return L["out"](o)
+            codes, rs = ops.hif8_gdn_decode_head_quant(
+                conv, qkvz, x, L["ba"], L["A_log"], L["dt_bias"], st.rec_states[idx], L["out_norm"],
+                L["out"].layer.input_scale, c.lin_k_heads, c.lin_v_heads, c.lin_k_dim, c.lin_v_dim, c.rms_eps)
+            return L["out"].from_codes(codes, rs)
         qkvz = L["qkvz"](x) if xq is None else L["qkvz"].from_codes(*xq)
         o = ops.hif8_gdn_decode_token(
             qkvz, x, L["ba"], L["conv"], st.conv_states[idx], L["A_log"], L["dt_bias"], st.rec_states[idx],

@@ -464,11 +464,29 @@ int hif8_gdn_decode_head(const float *conv, const uint16_t *mixed_qkvz, int64_t 
                          const uint16_t *ba_weight, int64_t hidden, const float *a_log, const float *dt_bias,
                          float *rec_state, const uint16_t *out_norm, uint16_t *out, int64_t batch, int64_t k_heads,
                          int64_t v_heads, int64_t k_dim, int64_t v_dim, float eps, hif8_stream_t stream);
+/* hif8_gdn_decode_head followed by hif8_static_quant of its output with the fixed
+ * scale input_scale[0], in one launch: the codes [batch, v_heads * v_dim] and
+ * row_scale [batch] of the out projection's input (the bf16 output is not stored). */
+int hif8_gdn_decode_head_quant(const float *conv, const uint16_t *mixed_qkvz, int64_t ld, const uint16_t *x,
+                               const uint16_t *ba_weight, int64_t hidden, const float *a_log, const float *dt_bias,
+                               float *rec_state, const uint16_t *out_norm, const float *input_scale, uint8_t *codes,
+                               float *row_scale, int64_t batch, int64_t k_heads, int64_t v_heads, int64_t k_dim,
+                               int64_t v_dim, float eps, hif8_stream_t stream);
 int hif8_qk_norm_rope(const uint16_t *qkv, const uint16_t *q_norm, const uint16_t *k_norm, const int64_t *pos,
                       const float *inv_freq, const int32_t *block_table, int64_t max_blocks, int64_t block_size,
                       uint16_t *q_out, uint16_t *k_out, uint16_t *v_out, int64_t *slots, int64_t batch,
                       int64_t num_heads, int64_t num_kv_heads, int64_t head_size, int64_t rotary_dim, float eps,
                       hif8_stream_t stream);
+/* hif8_qk_norm_rope followed by hif8_kv_cache_write of its k and v at its slots, in
+ * one launch: caches [num_blocks, block_size, num_kv_heads, head_size + 4], scales
+ * [num_kv_heads]; a position outside the block table or the cache writes nothing.
+ * head_size % 4 == 0 and <= 256. */
+int hif8_qk_norm_rope_cache(const uint16_t *qkv, const uint16_t *q_norm, const uint16_t *k_norm, const int64_t *pos,
+                            const float *inv_freq, const int32_t *block_table, int64_t max_blocks,
+                            int64_t num_blocks, int64_t block_size, uint16_t *q_out, uint8_t *key_cache,
+                            uint8_t *value_cache, const float *key_scale, const float *value_scale, int64_t batch,
+                            int64_t num_heads, int64_t num_kv_heads, int64_t head_size, int64_t rotary_dim,
+                            float eps, hif8_stream_t stream);
 int hif8_gdn_decode_step(const uint16_t *mixed_qkvz, int64_t ld, const uint16_t *ba,
                          const uint16_t *conv_weight, uint16_t *conv_state, const float *a_log,
                          const float *dt_bias, float *rec_state, const uint16_t *out_norm, uint16_t *out,

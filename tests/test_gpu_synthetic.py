@@ -455,3 +455,53 @@ def test_fused_attention_step_matches_torch_step(model, device):
         torch.testing.assert_close(st_a.key_caches[0], st_b.key_caches[0], rtol=0, atol=0)
         torch.testing.assert_close(st_a.value_caches[0], st_b.value_caches[0], rtol=0, atol=0)
         torch.testing.assert_close(fused.float(), ref.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("b,kh,vh,dk,dv,hidden", [(1, 16, 32, 128, 128, 4096), (3, 2, 4, 32, 32, 256),
+                                                  (2, 3, 3, 64, 96, 520)])
+def test_decode_head_quant_equals_head_then_static_quant(native_ops, device, b, kh, vh, dk, dv, hidden):
+    from hif8_rocm import native
+
+    ops = torch.ops.vllm_ascend_hif8
+    g = torch.Generator(device=device).manual_seed(b + dk)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device=device)
+
+    channels, bf = 2 * kh * dk + vh * dv, torch.bfloat16
+    args = [rand(b, channels), rand(b, channels + vh * dv).to(bf), rand(b, hidden).to(bf),
+            (rand(2 * vh, hidden) * 0.05).to(bf), rand(vh) * 0.5, rand(vh) * 0.5]
+    state = rand(b, vh, dk, dv) * 0.1
+    norm = torch.ones(dv, device=device, dtype=bf)
+    norm[0] = float("inf")  # one column of Inf, so codes of Inf too
+    scale = torch.tensor([0.07], device=device)
+    state_b = state.clone()
+    want = ops.hif8_gdn_decode_head(*args, state, norm, kh, vh, dk, dv, 1e-6)
+    codes, rs = ops.hif8_gdn_decode_head_quant(*args, state_b, norm, scale, kh, vh, dk, dv, 1e-6)
+    want_codes, want_rs = native.static_quant(want, scale)
+    assert torch.equal(codes, want_codes) and torch.equal(rs, want_rs) and torch.equal(state, state_b)
+
+
+@pytest.mark.parametrize("d,rot,bs", [(256, 64, 128), (64, 64, 16), (20, 8, 4)])
+def test_qk_norm_rope_cache_equals_rope_then_cache_write(native_ops, device, d, rot, bs):
+    """Also for positions past the table, blocks outside the cache (nothing
+    written) and the last slot."""
+    from hif8_rocm import kv_cache
+
+    ops = torch.ops.vllm_ascend_hif8
+    g = torch.Generator(device=device).manual_seed(d)
+    b, hq, hkv, blocks = 5, 4, 2, 6
+    qkv = (torch.randn(b, (hq + 2 * hkv) * d, generator=g, device=device) * 3).to(torch.bfloat16)
+    wq, wk = (torch.rand(d, generator=g, device=device).to(torch.bfloat16) + 0.5 for _ in range(2))
+    inv = 1.0 / 10000 ** (torch.arange(0, rot, 2, device=device).float() / rot)
+    table = torch.tensor([[0, 1], [2, 3], [4, 5], [blocks, 1], [5, -1]], dtype=torch.int32, device=device)
+    pos = torch.tensor([0, 2 * bs - 1, 2 * bs, 3, bs + 1], device=device)  # the last three write nothing
+    scales = [torch.rand(hkv, generator=g, device=device) * 0.01 + 1e-3 for _ in range(2)]
+    caches = [torch.zeros(blocks, bs, hkv, d + 4, dtype=torch.uint8, device=device) for _ in range(4)]
+    q, k, v, slots = ops.hif8_qk_norm_rope(qkv, wq, wk, pos, inv, table, bs, hq, hkv, d, 1e-6)
+    kv_cache.write_kv_cache(k, v, caches[0], caches[1], slots, *scales, validate=False)
+    got = ops.hif8_qk_norm_rope_cache(qkv, wq, wk, pos, inv, table, caches[2], caches[3], *scales, hq, 1e-6)
+    torch.cuda.synchronize()
+    assert torch.equal(got, q)
+    assert torch.equal(caches[2], caches[0]) and torch.equal(caches[3], caches[1])
+    assert int((caches[2] != 0).any(-1).sum()) == 2 * hkv
