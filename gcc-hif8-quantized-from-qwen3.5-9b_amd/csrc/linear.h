@@ -58,10 +58,9 @@ struct LinearArgs {
   GemvConv conv;                          // GEMV only: causal-conv epilogue
 };
 
-// HBM-streaming GEMV for m <= 4 (gemv.hip).  Returns a status; with a.pair
-// set, HIF8_ERR_UNSUPPORTED where the plan is not the dot2 kernel; with
-// a.conv set, HIF8_ERR_UNSUPPORTED where it is neither the dot2 nor the
-// MFMA-4 kernel.
+// HBM-streaming GEMV for m <= 4 (gemv.hip).  Returns a status; with a.pair or
+// a.conv set, HIF8_ERR_UNSUPPORTED where the plan is neither the dot2 nor the
+// MFMA-4 kernel (for a.pair one of 8 or 16 rows per block, and a.pair.inter % 8 == 0).
 int launch_gemv(const LinearArgs &a);
 // The conv epilogue of a.conv as a kernel of its own over y [m, ld] bf16 (the
 // projection output), for plans without the epilogue.

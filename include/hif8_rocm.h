@@ -433,8 +433,8 @@ int hif8_silu_mul_quant(const uint16_t *gate_up, const float *input_scale, uint8
  * channel_scale [2 inter] as for soft_hif8_gemm over activation codes [m, k]
  * with token_scale [m]; codes [m, inter] and row_scale [m] equal
  * hif8_silu_mul_quant(soft_hif8_gemm(...) in bf16, input_scale) bit for bit.
- * 1 <= m <= 4; HIF8_ERR_UNSUPPORTED where the GEMV plan for (m, 2 inter, k)
- * is not the dot2 kernel (then run the two calls). */
+ * 1 <= m <= 4; HIF8_ERR_UNSUPPORTED where no GEMV with this epilogue takes
+ * (m, 2 inter, k), e.g. k % 16 != 0 (then run the two calls). */
 int hif8_gate_up_silu_mul_quant(const uint8_t *activation, const uint8_t *weight, const float *token_scale,
                                 const float *channel_scale, const float *input_scale, uint8_t *codes,
                                 float *row_scale, int64_t m, int64_t inter, int64_t k, hif8_stream_t stream);

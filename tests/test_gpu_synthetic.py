@@ -214,9 +214,9 @@ def test_fused_add_rms_norm_silu_mul_and_bf16_gemv_match_torch(native_ops, devic
 def test_fused_gate_up_silu_mul_quant_equals_gemv_then_silu_mul_quant(m, inter, k, native_ops, device):
     """hif8_gate_up_silu_mul_quant: the gate_up GEMV whose blocks pair gate
     and up rows and finish with SiLU-mul and the static quant gives the codes
-    of soft_hif8_gemm (bf16) + SiLU-mul + static quant bit for bit (where the
-    GEMV plan is not the dot2 kernel, e.g. M = 4 over wide weights, the op
-    runs soft_hif8_gemm + hif8_silu_mul_quant itself)."""
+    of soft_hif8_gemm (bf16) + SiLU-mul + static quant bit for bit (where no
+    GEMV has the epilogue, e.g. K % 16 != 0, the op runs soft_hif8_gemm +
+    hif8_silu_mul_quant itself)."""
     ops = torch.ops.vllm_ascend_hif8
     g = torch.Generator(device=device).manual_seed(m * 7 + inter + k)
     w = torch.randn(2 * inter, k, generator=g, device=device).to(torch.bfloat16)
@@ -235,6 +235,31 @@ def test_fused_gate_up_silu_mul_quant_equals_gemv_then_silu_mul_quant(m, inter, 
         want, want_rs = native.static_quant(ops.hif8_silu_mul(gu), s)
         assert torch.equal(codes, want), (m, inter, k, sv)
         assert torch.equal(out_rs, want_rs.reshape(-1))
+
+
+@pytest.mark.parametrize("m,inter,k", [(3, 8192, 1040), (4, 8, 16), (4, 12, 64), (4, 6144, 4096), (4, 8200, 2064)])
+def test_mfma4_gate_up_silu_mul_quant_codes(m, inter, k, native_ops, device):
+    """The paired epilogue of the MFMA-4 GEMV (four rows, or three over wide
+    weights; blocks of 8 and 16 rows): codes and row scales equal the static
+    quant of the SiLU-mul of soft_hif8_gemm's bf16 outputs bit for bit.  A
+    width that is no multiple of 8 has no such epilogue and is refused."""
+    ops = torch.ops.vllm_ascend_hif8
+    from hif8_rocm import native
+    g = torch.Generator(device=device).manual_seed(m + inter + k)
+    w = torch.randn(2 * inter, k, generator=g, device=device).to(torch.bfloat16)
+    ws = (w.float().abs().amax(dim=1) / 32768.0).contiguous()
+    wq, _ = native.static_quant(w, ws)
+    x = torch.randn(m, k, generator=g, device=device).to(torch.bfloat16)
+    a, rs = native.static_quant(x, (x.float().abs().amax() / 32768.0).reshape(1))
+    a[m - 1, :3] = torch.tensor([0x80, 0x6F, 0xEF], dtype=torch.uint8, device=device)  # NaN, +Inf, -Inf codes
+    s = torch.tensor([0.01], device=device)
+    if inter % 8:
+        with pytest.raises(RuntimeError):
+            ops.hif8_gate_up_silu_mul_quant(a, wq, rs, ws, s)
+        return
+    codes, out_rs = ops.hif8_gate_up_silu_mul_quant(a, wq, rs, ws, s)
+    want, want_rs = native.static_quant(ops.hif8_silu_mul(ops.soft_hif8_gemm(a, wq, rs, ws, None, torch.bfloat16)), s)
+    assert torch.equal(codes, want) and torch.equal(out_rs, want_rs.reshape(-1))
 
 
 @pytest.mark.parametrize("shape", [
