@@ -20,14 +20,16 @@
 //     channel;
 //   * kDepth steps of both operands are in flight per wavefront.
 // What bounds it on MI355X: at M <= 32 over a wide weight the stream (24576 x
-// 4096 at M = 16: 33 us with the decode launch, 3.6 TB/s; the 128 x 128 tiles,
+// 4096 at M = 16: 32.2 us with the decode launch, 3.6 TB/s; the 128 x 128 tiles,
 // which decode W into LDS behind a barrier per step: 52 us); over narrow ones
 // the two launches and the wavefront's chain of loads (2048 x 4096: 9.6 vs
 // 22.5 us); from M = 48 on the fragment reads, M / 16 KiB per 64 x 16 codes
 // through the vector cache (24576 x 4096: M = 64 44.6 us).  Read row-major the
 // same fragments took 41.8 us at M = 32 instead of 36.5 and 61.6 at M = 64.
-// Deeper pipelines (3, 4 steps), 16 wavefronts and a start rotated per block
-// measured the same or slower.
+// The padding rows of the last fragment are not read: 4096 x 12288 at M = 5
+// 22.6 -> 18.7 us, M = 24 26.6 -> 24.4.  Deeper pipelines (3, 4 steps), 16
+// wavefronts, 64 weight rows per block (24576 x 4096 at M = 24: 38 us) and a
+// start rotated per block measured the same or slower.
 // K need not be a multiple of anything and weight rows need no alignment (the
 // loads are emitted for byte alignment): the one partial step masks its codes
 // to zero, and the bf16 copy is zero-padded to a multiple of 64.
@@ -78,14 +80,19 @@ __global__ __launch_bounds__(kWave * kWaves) void gemm_skinny_kernel(
 
   for (int i = tid; i < 256; i += kWave * kWaves) lut[i] = uint16_t(decode_bits(uint32_t(i)) >> 16);
 
-  // Rows past the end re-read the last one; their sums are not stored.
+  // Rows past the end re-read the last one; their sums are not stored.  For the
+  // activation this leaves the cache lines of a fragment's padding rows alone
+  // (eight rows of a fragment are one line).
   const uint8_t *wrow[kNT];
   const u32x4 *afrag[kMT];
 #pragma unroll
   for (int j = 0; j < kNT; ++j) wrow[j] = W + size_t(min(n0 + 16 * j + frow, N - 1)) * K + 16 * fgrp;
 #pragma unroll
-  for (int i = 0; i < kMT; ++i)
-    afrag[i] = reinterpret_cast<const u32x4 *>(A) + size_t(min(m0 / 16 + i, (M - 1) / 16)) * steps * 2 * kWave + lane;
+  for (int i = 0; i < kMT; ++i) {
+    const int tile = min(m0 / 16 + i, (M - 1) / 16);
+    afrag[i] = reinterpret_cast<const u32x4 *>(A) + size_t(tile) * steps * 2 * kWave + 16 * fgrp +
+               min(frow, M - 1 - 16 * tile);
+  }
 
   struct Stage {
     u32x4 a[kMT][2], w[kNT];
@@ -285,12 +292,15 @@ int launch_gemm_skinny(const LinearArgs &a, const uint16_t *act) {
   // 32 weight rows per block share the activation fragments of a step (wide N,
   // or row tiles that fill the CUs); otherwise 16 give more CUs a block, and
   // eight wavefronts each a shorter chain.  MI355X, with the decode launch:
-  // 24576 x 4096 at M = 24 36.5 us (16 rows per block: 44), M = 64 44.6 (59);
-  // 2048 x 4096 at M = 24 11.5 (32 rows per block: 14.1), M = 64 14.5 (17.2).
+  // 24576 x 4096 at M = 24 34.2 us (16 rows per block: 39.8), M = 64 44.9 (58.5);
+  // 2048 x 4096 at M = 24 10.6 (32 rows per block: 13.0), M = 64 14.5 (17.9).
   const bool wide = (a.n + 15) / 16 * ((a.m + 63) / 64) > 256;
+  // Eight wavefronts in the wide blocks too while the sums of up to 32 rows leave
+  // their meeting place small (8192 x 4096: M = 5 13.5 us, four wavefronts 14.9;
+  // 24576 x 4096: M = 24 34.2 against 35.2, but M = 40 41.4 against 39.0).
   switch (std::min<int64_t>((a.m + 15) / 16, 4)) {
-    case 1: return wide ? launch_skinny_t<1, 2, 4, 2>(a, act, steps) : launch_skinny_t<1, 1, 8, 2>(a, act, steps);
-    case 2: return wide ? launch_skinny_t<2, 2, 4, 2>(a, act, steps) : launch_skinny_t<2, 1, 8, 2>(a, act, steps);
+    case 1: return wide ? launch_skinny_t<1, 2, 8, 2>(a, act, steps) : launch_skinny_t<1, 1, 8, 2>(a, act, steps);
+    case 2: return wide ? launch_skinny_t<2, 2, 8, 2>(a, act, steps) : launch_skinny_t<2, 1, 8, 2>(a, act, steps);
     case 3: return wide ? launch_skinny_t<3, 2, 4, 2>(a, act, steps) : launch_skinny_t<3, 1, 8, 2>(a, act, steps);
     default: return wide ? launch_skinny_t<4, 2, 4, 2>(a, act, steps) : launch_skinny_t<4, 1, 8, 2>(a, act, steps);
   }
