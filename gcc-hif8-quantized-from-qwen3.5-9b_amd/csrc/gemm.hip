@@ -41,7 +41,6 @@ namespace hif8 {
 namespace {
 
 constexpr int kBK = 64;  // bytes (= bf16 elements) of K per stage
-constexpr int64_t kMaxSkinnyK = 0x7FFFFF00ll;  // k rounded up to 64 fits int
 constexpr int kMaxDmaK = 1 << 23;  // gemm_dma_kernel: a tile's rows in 32-bit byte offsets
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -1083,7 +1082,6 @@ int launch_prepared(const LinearArgs &a, const GemmPlan &p, uint8_t *ws) {
 // x 4096 15.4 vs 25.3; M = 128 4096 x 4096 18.5 vs 28.6; M = 256 2048 x 4096
 // 18.1 vs 27.9; but M = 128 4096 x 12288 43 vs 37.7 and 24576 x 4096 70 vs 59.
 bool skinny_rule(int64_t m, int64_t n, int64_t k) {
-  if (k > kMaxSkinnyK) return false;
   return k % kBK != 0 || m <= 64 || (k <= 8192 && (n + 31) / 32 * ((m + 63) / 64) <= 256);
 }
 
@@ -1103,7 +1101,7 @@ size_t gemm_scratch_size(int64_t m, int64_t n, int64_t k) {
   // per wavefront (MI355X, a scheme call in a graph, 4 x 2900 x 4100 97.4 ->
   // 17.3 us, 1 x 1000 x 2052 31.6 -> 14.6, 1 x 60 x 100 16.8 -> 13.8).
   if (m <= 4 && k % 16 == 0) return 0;
-  return k % kBK ? (skinny_rule(m, n, k) ? skinny_workspace_size(m, k) : 0) : gemm_workspace_size(m, n, k);
+  return k % kBK ? skinny_workspace_size(m, k) : gemm_workspace_size(m, n, k);
 }
 
 int launch_gemm(const LinearArgs &a) {
@@ -1142,7 +1140,7 @@ int launch_gemm(const LinearArgs &a) {
 }
 
 size_t gemm_static_workspace_size(int64_t m, int64_t n, int64_t k) {
-  if (m <= 0 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > kMaxSkinnyK || n <= 0 || k <= 0) return 0;
+  if (m <= 0 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > 0x7FFFFFFFll || n <= 0 || k <= 0) return 0;
   if (m <= 4 && k % 16 == 0) return 0;  // the GEMV's
   const size_t scales = (size_t(m) * sizeof(float) + 255) / 256 * 256;
   // Fragments also where a weight that is not 16-byte aligned keeps the tiles away.

@@ -35,6 +35,7 @@
 // to zero, and the bf16 copy is zero-padded to a multiple of 64.
 #include <algorithm>
 
+#include "fragment_layout.h"
 #include "gemm_operand.h"
 
 namespace hif8 {
@@ -44,8 +45,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_bytes __attribute__((aligned(1)));
-
-constexpr int kStepK = 64;
 
 // 16 codes -> 16 bf16 (lo = codes 0..7, hi = codes 8..15).
 __device__ __forceinline__ void decode16(const uint16_t *lut, const u32x4 q, u32x4 &lo, u32x4 &hi) {
@@ -90,8 +89,8 @@ __global__ __launch_bounds__(kWave * kWaves) void gemm_skinny_kernel(
 #pragma unroll
   for (int i = 0; i < kMT; ++i) {
     const int tile = min(m0 / 16 + i, (M - 1) / 16);
-    afrag[i] = reinterpret_cast<const u32x4 *>(A) + size_t(tile) * steps * 2 * kWave + 16 * fgrp +
-               min(frow, M - 1 - 16 * tile);
+    afrag[i] = reinterpret_cast<const u32x4 *>(A) +
+               fragment_word(tile, steps, 0, 0, 16 * fgrp + min(frow, M - 1 - 16 * tile));
   }
 
   struct Stage {
@@ -102,7 +101,7 @@ __global__ __launch_bounds__(kWave * kWaves) void gemm_skinny_kernel(
   auto load = [&](Stage &s, int k0) {
 #pragma unroll
     for (int t = 0; t < kMT; ++t) {
-      const u32x4 *p = afrag[t] + k0 / kStepK * 2 * kWave;
+      const u32x4 *p = afrag[t] + fragment_word(0, 0, k0 / kStepK, 0, 0);
       s.a[t][0] = p[0];
       s.a[t][1] = p[kWave];
     }
@@ -166,7 +165,7 @@ __global__ __launch_bounds__(kWave * kWaves) void gemm_skinny_kernel(
     Stage s;
 #pragma unroll
     for (int t = 0; t < kMT; ++t) {
-      const u32x4 *p = afrag[t] + k0 / kStepK * 2 * kWave;
+      const u32x4 *p = afrag[t] + fragment_word(0, 0, k0 / kStepK, 0, 0);
       s.a[t][0] = p[0];
       s.a[t][1] = p[kWave];
     }
@@ -252,8 +251,8 @@ __global__ __launch_bounds__(256) void decode_fragments_kernel(const uint8_t *__
     }
     u32x4 lo, hi;
     decode16(lut, q, lo, hi);
-    out[frag * 2 * kWave + lane] = lo;
-    out[frag * 2 * kWave + kWave + lane] = hi;
+    out[fragment_word(0, 0, frag, 0, lane)] = lo;
+    out[fragment_word(0, 0, frag, 1, lane)] = hi;
   }
 }
 

@@ -235,7 +235,7 @@ extern "C" int hif8_static_linear(const void *x, int x_dtype, const uint8_t *wei
   if (!is_io_dtype(x_dtype))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "activation must have dtype torch.float16 or torch.bfloat16");
   const size_t need = gemm_static_workspace_size(m, n, k);
-  if (need == 0) return fail(HIF8_ERR_UNSUPPORTED, "hif8_static_linear requires M > 4 or K %% 16 != 0, and K < 2^31 - 256");
+  if (need == 0) return fail(HIF8_ERR_UNSUPPORTED, "hif8_static_linear requires M > 4 or K %% 16 != 0");
   if (!workspace || workspace_bytes < need || !aligned(workspace, 256))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_static_linear: needs a 256-byte aligned workspace of %zu bytes", need);
   LinearArgs a = codes_args(nullptr, weight, fixed_scale, channel_scale, bias, bias_dtype, out, out_dtype, m, n, k,

@@ -6,6 +6,7 @@
 // instead of 5.2 + 4.9 on average, of 4096 rows 21 us (4.5 TB/s).
 #include <algorithm>
 
+#include "fragment_layout.h"
 #include "gemm_operand.h"
 #include "qdq_device.h"
 
@@ -15,7 +16,6 @@ namespace {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kStepK = 64;
 
 // kFrag: the fragment order of gemm_skinny_kernel, rows padded to 16 and k to
 // 64 with zeros; otherwise row-major.  kVec: k % 16 == 0 and 16-byte aligned x
@@ -89,9 +89,8 @@ __global__ __launch_bounds__(kThreads) void static_operand_kernel(const uint16_t
     }
     const u32x4 lo = {p[0], p[1], p[2], p[3]}, hi = {p[4], p[5], p[6], p[7]};
     if constexpr (kFrag) {
-      const int64_t at = item / kWave * 2 * kWave + item % kWave;
-      out[at] = lo;
-      out[at + kWave] = hi;
+      out[fragment_word(0, 0, item / kWave, 0, int(item % kWave))] = lo;
+      out[fragment_word(0, 0, item / kWave, 1, int(item % kWave))] = hi;
     } else {
       out[2 * item] = lo;
       out[2 * item + 1] = hi;

@@ -136,6 +136,24 @@ def test_few_row_and_ragged_gemm(native_ops, device, rows, channels, k):
     _check(y[:, torch.from_numpy(keep).to(device)], want)
 
 
+@pytest.mark.parametrize("rows,k", [(1, 2 ** 30 + 65), (5, 2 ** 30 + 64)])
+def test_few_row_gemm_of_rows_beyond_32_bit_offsets(native_ops, device, rows, k):
+    """Activation rows of more than 2^30 codes (fragment offsets past 32 bits):
+    non-zero only in a few places, on both sides of 2^30 and at the end."""
+    rng = np.random.default_rng(rows)
+    at = np.unique(np.concatenate([[0, 2 ** 30 - 1, 2 ** 30, 2 ** 30 + 63, k - 1], rng.integers(0, k, 40)]))
+    codes, weights = random_codes((rows, at.size), seed=rows), random_codes((2, at.size), seed=7)
+    act = torch.zeros(rows, k, dtype=torch.uint8, device=device)
+    weight = torch.full((2, k), int(o.encode_scalar(1.0)), dtype=torch.uint8, device=device)
+    where = torch.from_numpy(at).to(device)
+    act[:, where] = _t(codes, device)
+    weight[:, where] = _t(weights, device)
+    ts, cs = np.full(rows, 1e-3, np.float32), np.full(2, 1e-3, np.float32)
+    y = native_ops.soft_hif8_gemm(act, weight, _t(ts, device), _t(cs, device), None, torch.bfloat16)
+    torch.cuda.synchronize()
+    _check(y, o.linear_u8_u8(codes, ts, weights, cs, None))
+
+
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320])
 @pytest.mark.parametrize("rows,channels", [(300, 11001), (500, 22024)])
 def test_weight_decoding_tiles_of_few_steps(native_ops, device, rows, channels, k):
