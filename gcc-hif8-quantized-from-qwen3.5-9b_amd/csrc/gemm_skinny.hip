@@ -63,15 +63,16 @@ template <int kMT, int kNT, int kWaves, int kDepth>
 __global__ __launch_bounds__(kWave * kWaves) void gemm_skinny_kernel(
     const uint16_t *__restrict__ A, int steps, const float *__restrict__ ts, const uint8_t *__restrict__ W,
     const float *__restrict__ cs, const void *__restrict__ bias, int bias_dtype, void *__restrict__ out,
-    int out_dtype, int M, int N, int K, int n_tiles, int m_tiles) {
+    int out_dtype, int M, int N, int K, int n_tiles, int m_tiles, int n_first, int m_first) {
   constexpr int kBM = 16 * kMT, kBN = 16 * kNT;
   __shared__ __attribute__((aligned(16))) uint16_t lut[256];
   __shared__ __attribute__((aligned(16))) f32x4_t red[kWaves][kNT][kMT][kWave];
 
-  // The row tiles that read the same weight rows are 8 block ids apart: one
-  // XCD, whose L2 then serves all but the first.
+  // The row tiles (m_tiles of this launch, from m_first on) that read the same
+  // weight rows are 8 block ids apart: one XCD, whose L2 then serves all but the
+  // first.
   const int group = int(blockIdx.x) / (8 * m_tiles), in_group = int(blockIdx.x) - group * 8 * m_tiles;
-  const int nt = group * 8 + (in_group & 7), mt = in_group >> 3;
+  const int nt = n_first + group * 8 + (in_group & 7), mt = m_first + (in_group >> 3);
   if (nt >= n_tiles) return;
   const int n0 = nt * kBN, m0 = mt * kBM;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -259,12 +260,19 @@ __global__ __launch_bounds__(256) void decode_fragments_kernel(const uint8_t *__
 template <int kMT, int kNT, int kWaves, int kDepth>
 int launch_skinny_t(const LinearArgs &a, const uint16_t *act, int steps) {
   const int64_t n_tiles = (a.n + 16 * kNT - 1) / (16 * kNT), m_tiles = (a.m + 16 * kMT - 1) / (16 * kMT);
-  const int64_t blocks = (n_tiles + 7) / 8 * 8 * m_tiles;
-  if (blocks > 0x7FFFFFFFll) return fail(HIF8_ERR_UNSUPPORTED, "soft_hif8 GEMM: too many tiles");
-  gemm_skinny_kernel<kMT, kNT, kWaves, kDepth><<<unsigned(blocks), kWave * kWaves, 0, a.stream>>>(
-      act, steps, a.act_scale, a.weight, a.channel_scale, a.bias, a.bias_dtype, a.out, a.out_dtype, int(a.m),
-      int(a.n), int(a.k), int(n_tiles), int(m_tiles));
-  return check_launch("soft_hif8 GEMM (few rows)");
+  // A launch holds fewer than 2^32 threads; more tiles go in several.
+  constexpr int64_t kMaxBlocks = 0xFFFFFFFFll / (kWave * kWaves);
+  const int64_t m_step = std::min(m_tiles, kMaxBlocks / 8), n_step = kMaxBlocks / (8 * m_step) * 8;
+  for (int64_t nf = 0; nf < n_tiles; nf += n_step) {
+    for (int64_t mf = 0; mf < m_tiles; mf += m_step) {
+      const int64_t nb = (std::min(n_step, n_tiles - nf) + 7) / 8 * 8, mb = std::min(m_step, m_tiles - mf);
+      gemm_skinny_kernel<kMT, kNT, kWaves, kDepth><<<unsigned(nb * mb), kWave * kWaves, 0, a.stream>>>(
+          act, steps, a.act_scale, a.weight, a.channel_scale, a.bias, a.bias_dtype, a.out, a.out_dtype, int(a.m),
+          int(a.n), int(a.k), int(n_tiles), int(mb), int(nf), int(mf));
+      if (const int st = check_launch("soft_hif8 GEMM (few rows)")) return st;
+    }
+  }
+  return HIF8_OK;
 }
 
 }  // namespace

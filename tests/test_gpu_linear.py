@@ -154,6 +154,23 @@ def test_few_row_gemm_of_rows_beyond_32_bit_offsets(native_ops, device, rows, k)
     _check(y, o.linear_u8_u8(codes, ts, weights, cs, None))
 
 
+@pytest.mark.parametrize("rows,channels,k", [(5, 2 ** 28 + 2 ** 20 + 17, 3), (2 ** 27 + 2 ** 20 + 5, 3, 1)])
+def test_few_row_gemm_of_more_tiles_than_one_launch_holds(native_ops, device, rows, channels, k):
+    """More weight rows, or activation rows, than the threads of one launch (2^32)
+    cover: every output against a float32 product, which is exact for these codes."""
+    codes = torch.tensor([o.encode_scalar(float(v)) for v in (0, 1, -2, 3, 0.5)], dtype=torch.uint8, device=device)
+    values = torch.tensor([0.0, 1.0, -2.0, 3.0, 0.5], device=device)
+    g = torch.Generator(device=device).manual_seed(3)
+    at = [torch.randint(0, 5, s, generator=g, device=device, dtype=torch.uint8) for s in ((rows, k), (channels, k))]
+    act, weight = (codes[i.int()] for i in at)
+    ts, cs = torch.ones(rows, device=device), torch.ones(channels, device=device)
+    y = native_ops.soft_hif8_gemm(act, weight, ts, cs, None, torch.bfloat16)
+    torch.cuda.synchronize()
+    a, w = (values[i.int()] for i in at)
+    want = sum(a[:, j, None] * w[None, :, j] for j in range(k))
+    assert torch.equal(y.float(), want)
+
+
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320])
 @pytest.mark.parametrize("rows,channels", [(300, 11001), (500, 22024)])
 def test_weight_decoding_tiles_of_few_steps(native_ops, device, rows, channels, k):
