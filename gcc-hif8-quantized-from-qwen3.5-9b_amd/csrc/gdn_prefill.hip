@@ -413,8 +413,9 @@ __global__ __launch_bounds__(256) void conv_tokens_kernel(const uint16_t *__rest
 __global__ __launch_bounds__(256) void gated_norm_kernel(const float *__restrict__ o, int64_t ob, int64_t ot,
                                                          int64_t oh, const uint16_t *__restrict__ z, int64_t z_ld,
                                                          const uint16_t *__restrict__ w, uint16_t *__restrict__ out,
-                                                         int tokens, int heads, int dv, int64_t rows, float eps) {
-  const int64_t row = int64_t(blockIdx.x) * 4 + threadIdx.x / kWave;  // (b, t, h)
+                                                         int tokens, int heads, int dv, int64_t first, int64_t rows,
+                                                         float eps) {
+  const int64_t row = first + int64_t(blockIdx.x) * 4 + threadIdx.x / kWave;  // (b, t, h)
   if (row >= rows) return;
   const int lane = threadIdx.x % kWave;
   const int64_t bt = row / heads;
@@ -547,9 +548,15 @@ extern "C" int hif8_gated_rms_norm(const float *o, int64_t o_batch, int64_t o_to
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_gated_rms_norm: invalid dimensions");
   const int64_t rows = batch * tokens * heads;
   if (v_dim > 256 || v_dim % 2 || z_ld % 2 || o_batch % 2 || o_token % 2 || o_head % 2 || !aligned(o, 8) ||
-      !aligned(z, 4) || !aligned(weight, 4) || !aligned(out, 4) || rows > 4 * 0x7FFFFFFFll)
+      !aligned(z, 4) || !aligned(weight, 4) || !aligned(out, 4))
     return fail(HIF8_ERR_UNSUPPORTED, "hif8_gated_rms_norm: needs even v_dim <= 256, even strides and aligned rows");
-  gated_norm_kernel<<<unsigned((rows + 3) / 4), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
-      o, o_batch, o_token, o_head, z, z_ld, weight, out, int(tokens), int(heads), int(v_dim), rows, eps);
-  return check_launch("hif8_gated_rms_norm");
+  // A launch holds fewer than 2^32 threads.
+  constexpr int64_t kStep = int64_t(1) << 24;
+  for (int64_t first = 0; first < rows; first += kStep) {
+    gated_norm_kernel<<<unsigned((std::min(kStep, rows - first) + 3) / 4), 256, 0,
+                        reinterpret_cast<hipStream_t>(stream)>>>(o, o_batch, o_token, o_head, z, z_ld, weight, out,
+                                                                 int(tokens), int(heads), int(v_dim), first, rows, eps);
+    if (const int st = check_launch("hif8_gated_rms_norm")) return st;
+  }
+  return HIF8_OK;
 }

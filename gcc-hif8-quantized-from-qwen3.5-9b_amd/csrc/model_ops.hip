@@ -886,7 +886,8 @@ extern "C" int hif8_qk_norm_rope(const uint16_t *qkv, const uint16_t *q_norm, co
   if (!qkv || !q_norm || !k_norm || !pos || !inv_freq || !q_out || !k_out || !v_out || (slots && !block_table))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope: null pointer argument");
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||
-      rotary_dim < 0 || rotary_dim > head_size || rotary_dim % 2 || block_size <= 0 || batch > 65536)
+      rotary_dim < 0 || rotary_dim > head_size || rotary_dim % 2 || block_size <= 0 || batch > 65536 ||
+      batch * (num_heads + 2 * num_kv_heads) >= (int64_t(1) << 32) / kHeadThreads)
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope: unsupported dimensions");
   qk_norm_rope_kernel<false><<<unsigned(batch * (num_heads + 2 * num_kv_heads)), kHeadThreads, 0,
                                reinterpret_cast<hipStream_t>(stream)>>>(
@@ -908,7 +909,8 @@ extern "C" int hif8_qk_norm_rope_cache(const uint16_t *qkv, const uint16_t *q_no
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope_cache: null pointer argument");
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||
       head_size % 4 || rotary_dim < 0 || rotary_dim > head_size || rotary_dim % 2 || block_size <= 0 ||
-      block_size > 0x7FFFFFFFll || num_blocks <= 0 || batch > 65536 || !aligned(key_cache, 4) ||
+      block_size > 0x7FFFFFFFll || num_blocks <= 0 || batch > 65536 ||
+      batch * (num_heads + 2 * num_kv_heads) >= (int64_t(1) << 32) / kHeadThreads || !aligned(key_cache, 4) ||
       !aligned(value_cache, 4))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope_cache: unsupported dimensions");
   CacheRows cache;
@@ -933,15 +935,23 @@ extern "C" int hif8_add_rms_norm(uint16_t *h, const uint16_t *delta, const uint1
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool vec = n % 8 == 0 && n <= 8 * kRowThreads * kRowChunks && aligned(h, 16) && aligned(weight, 16) &&
                    aligned(out, 16) && (!delta || aligned(delta, 16));
-  if (vec && delta)
-    add_rms_norm_vec_kernel<true><<<unsigned(rows), kRowThreads, 0, s>>>(h, delta, weight, out, int(n), eps);
-  else if (vec)
-    add_rms_norm_vec_kernel<false><<<unsigned(rows), kRowThreads, 0, s>>>(h, nullptr, weight, out, int(n), eps);
-  else if (delta)
-    add_rms_norm_kernel<true><<<unsigned(rows), kNormThreads, 0, s>>>(h, delta, weight, out, int(n), eps);
-  else
-    add_rms_norm_kernel<false><<<unsigned(rows), kNormThreads, 0, s>>>(h, nullptr, weight, out, int(n), eps);
-  return check_launch("hif8_add_rms_norm");
+  // A launch holds fewer than 2^32 threads.
+  constexpr int64_t kStep = int64_t(1) << 22;
+  for (int64_t first = 0; first < rows; first += kStep) {
+    const unsigned blocks = unsigned(std::min(kStep, rows - first));
+    uint16_t *hr = h + first * n, *orow = out + first * n;
+    const uint16_t *dr = delta ? delta + first * n : nullptr;
+    if (vec && delta)
+      add_rms_norm_vec_kernel<true><<<blocks, kRowThreads, 0, s>>>(hr, dr, weight, orow, int(n), eps);
+    else if (vec)
+      add_rms_norm_vec_kernel<false><<<blocks, kRowThreads, 0, s>>>(hr, dr, weight, orow, int(n), eps);
+    else if (delta)
+      add_rms_norm_kernel<true><<<blocks, kNormThreads, 0, s>>>(hr, dr, weight, orow, int(n), eps);
+    else
+      add_rms_norm_kernel<false><<<blocks, kNormThreads, 0, s>>>(hr, dr, weight, orow, int(n), eps);
+    if (const int st = check_launch("hif8_add_rms_norm")) return st;
+  }
+  return HIF8_OK;
 }
 
 extern "C" int hif8_add_rms_norm_quant(uint16_t *h, const uint16_t *delta, const uint16_t *weight, uint16_t *out,

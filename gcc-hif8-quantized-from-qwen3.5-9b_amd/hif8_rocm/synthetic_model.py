@@ -401,7 +401,7 @@ class HybridModel:
         c = self.cfg
         b, t, _ = h.shape
         qkv = L["qkv"](h.reshape(b * t, -1)).reshape(b, t, -1)
-        if not decode and c.head_dim <= 256 and b * t <= 65536:
+        if not decode and self._rope_kernel(b * t):
             # Row i of the fused kernel is one token: norms, rotary and the split
             # in one launch (its cache slots are not used: _slots below checks them).
             q, k, v, _ = torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope(
@@ -452,7 +452,7 @@ class HybridModel:
         gdecay = -torch.exp(L["A_log"]) * torch.nn.functional.softplus(ba[..., c.lin_v_heads:] + L["dt_bias"])
         # Causal depthwise conv over time with the carried state (width conv_kernel).
         conv_state = st.conv_states[idx]
-        if self._prefill_kernels(t):
+        if self._prefill_kernels(b, t):
             mixed = torch.ops.vllm_ascend_hif8.hif8_conv_tokens(qkvz, L["conv"], conv_state)
         else:
             seq = torch.cat([conv_state, mixed.transpose(1, 2)], dim=-1)       # [B, C, K-1+T]
@@ -474,7 +474,7 @@ class HybridModel:
             rule = gated_delta_chunked if self.delta_kernel else _gated_delta_torch
             o = rule(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2),
                      gdecay.transpose(1, 2), beta.transpose(1, 2), state).transpose(1, 2)
-        if self._prefill_kernels(t):
+        if self._prefill_kernels(b, t):
             o = torch.ops.vllm_ascend_hif8.hif8_gated_rms_norm(o, qkvz, 2 * c.lin_qk_width + c.lin_v_width,
                                                                L["out_norm"], c.rms_eps)
             return L["out"](o.reshape(b * t, c.lin_v_width)).reshape(b, t, -1)
@@ -483,10 +483,15 @@ class HybridModel:
         o = o.to(h.dtype).reshape(b * t, c.lin_v_width)
         return L["out"](o).reshape(b, t, -1)
 
-    def _prefill_kernels(self, t: int) -> bool:
-        """Whether the glue kernels of a prefill take these sizes (t: tokens per request)."""
+    def _rope_kernel(self, rows: int) -> bool:
+        """Whether hif8_qk_norm_rope takes these token rows in one launch."""
         c = self.cfg
-        return (2 <= c.conv_kernel <= 4 and (2 * c.lin_qk_width + c.lin_v_width) % 2 == 0 and c.lin_v_dim % 2 == 0
+        return c.head_dim <= 256 and rows <= 65536 and rows * (c.heads + 2 * c.kv_heads) < 1 << 24
+
+    def _prefill_kernels(self, b: int, t: int) -> bool:
+        """Whether the glue kernels of a prefill take these sizes (b requests of t tokens)."""
+        c = self.cfg
+        return (b <= 65535 and 2 <= c.conv_kernel <= 4 and (2 * c.lin_qk_width + c.lin_v_width) % 2 == 0 and c.lin_v_dim % 2 == 0
                 and c.lin_v_dim <= 256 and 0 < t <= 1 << 19)
 
     def _linear_attention_decode(self, L, idx: int, st: RequestState, x: torch.Tensor, xq=None) -> torch.Tensor:

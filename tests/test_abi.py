@@ -186,3 +186,12 @@ def test_prefill_attention_contract_and_workspace_plan(lib):
     assert call(query=None) == 1 and b"null pointer" in lib.hif8_last_error()
     assert call() == 1 and b"workspace of" in lib.hif8_last_error()
     assert call(ws=_p(264), ws_bytes=1 << 30) == 1 and b"16-byte aligned" in lib.hif8_last_error()
+
+
+def test_qk_norm_rope_rejects_more_blocks_than_a_launch_holds(lib):
+    f = lib.hif8_qk_norm_rope
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+    f.argtypes = [ptr] * 6 + [i64] * 2 + [ptr] * 4 + [i64] * 5 + [ctypes.c_float, ptr]
+    for heads in (248, 1 << 20):
+        assert f(*[_p(16)] * 6, 4, 16, *[_p(16)] * 4, 65536, heads, 4, 64, 64, 1e-6, None) == 1
+        assert b"unsupported dimensions" in lib.hif8_last_error()

@@ -95,6 +95,23 @@ def test_gated_rms_norm_matches_torch(native_ops, device, b, t, h, dv, offset):
     torch.testing.assert_close(got.double(), want.reshape(b, t, -1), rtol=2 ** -8 + 1e-5, atol=1e-30)
 
 
+def test_norms_of_more_rows_than_one_launch_holds(native_ops, device):
+    """Rows past the 2^32 threads of one launch: the last ones equal a call of their own."""
+    ops, g = torch.ops.vllm_ascend_hif8, torch.Generator(device=device).manual_seed(5)
+    bf, rows, n = torch.bfloat16, 2 ** 23 + 9, 8
+    h = torch.randn(rows, n, generator=g, device=device).to(bf)
+    w = torch.rand(n, generator=g, device=device).to(bf)
+    tail_h, delta = h[-40:].clone(), h.flip(0).contiguous()
+    want, got = (ops.hif8_add_rms_norm(x, d, w, 1e-6) for x, d in ((tail_h, delta[-40:].contiguous()), (h, delta)))
+    assert torch.equal(got[-40:], want) and torch.equal(h[-40:], tail_h)
+    tokens = 2 ** 26 + 9
+    o = torch.randn(1, tokens, 1, 2, generator=g, device=device)
+    mixed = torch.randn(1, tokens, 2, generator=g, device=device).to(bf)
+    got = ops.hif8_gated_rms_norm(o, mixed, 0, w[:2].contiguous(), 1e-6)
+    want = ops.hif8_gated_rms_norm(o[:, -40:].contiguous(), mixed[:, -40:].contiguous(), 0, w[:2].contiguous(), 1e-6)
+    assert torch.equal(got[:, -40:], want)
+
+
 @pytest.mark.parametrize("rows,n", [(1, 8), (3, 24), (5, 6), (300, 1024)])
 def test_silu_mul_equals_torch(native_ops, device, rows, n):
     g = torch.Generator().manual_seed(n)

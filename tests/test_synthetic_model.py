@@ -6,7 +6,7 @@ that is not a multiple of the chunk."""
 import pytest
 import torch
 
-from hif8_rocm.synthetic_model import HybridConfig, gated_delta_chunked, gated_delta_step
+from hif8_rocm.synthetic_model import HybridConfig, HybridModel, gated_delta_chunked, gated_delta_step
 
 
 def _inputs(b, h, t, dk, dv, seed):
@@ -48,3 +48,14 @@ def test_config_follows_the_hybrid_layout():
     assert full == [3, 7, 11, 15, 19, 23, 27, 31]
     assert c.lin_v_width == 4096 and c.intermediate == 12288 and c.hidden == 4096
     assert (c.heads + 2 * c.kv_heads) * c.head_dim == 4096 + 2048
+
+
+def test_prefill_kernels_are_left_where_a_launch_ends():
+    """Sizes past one launch of the glue kernels (2^32 threads, 65535 requests) stay in torch."""
+    model = HybridModel.__new__(HybridModel)
+    model.cfg = HybridConfig()
+    assert model._prefill_kernels(65535, 4) and not model._prefill_kernels(65536, 4)
+    assert model._prefill_kernels(1, 1 << 19) and not model._prefill_kernels(1, (1 << 19) + 1)
+    assert model._rope_kernel(65536) and not model._rope_kernel(65537)
+    model.cfg = HybridConfig(heads=248, kv_heads=4)
+    assert model._rope_kernel(65535) and not model._rope_kernel(65536)
