@@ -890,9 +890,6 @@ int64_t image_cap_bytes() {
 struct PrefillPlans {
   PrefillPlan in, img;
   int slots, long_rows, img_tiles;
-  // As far as the totals tell, every request is as long as the longest and has a
-  // slot, so that the in-kernel path will find none of its own.
-  bool expect_no_short;
 };
 
 PrefillPlans plan_prefill(int64_t batch, int64_t hkv, int64_t group, int64_t total_q, int64_t max_query_len,
@@ -915,7 +912,6 @@ PrefillPlans plan_prefill(int64_t batch, int64_t hkv, int64_t group, int64_t tot
   const int64_t in_cover =
       pp.slots > 0 && pp.slots >= long_max ? std::min<int64_t>(max_query_len, pp.long_rows / group) : max_query_len;
   pp.in = plan_path(batch, hkv, group, in_cover, max_len, false);
-  pp.expect_no_short = pp.slots > 0 && pp.slots >= long_max && total_q >= batch * max_query_len;
   return pp;
 }
 
@@ -1119,13 +1115,6 @@ extern "C" int hif8_paged_prefill_attention(const void *query, int q_dtype, cons
         p.part_o = reinterpret_cast<float *>(ws + w.images + w.img_parts);
         p.part_ml = p.part_o + size_t(batch) * p.q_tiles * num_kv_heads * p.num_splits * kPRows * head_size_v;
       }
-    }
-    if (pp.expect_no_short) {
-      // Launched all the same for requests that the totals hide, but unsplit: its
-      // combine launch would find nothing either (MI355X, 4 x 512 rows over 4096
-      // keys 169.8 -> 167.9 us).
-      p.num_splits = 1;
-      p.split_tiles = int((max_seq_len + kKT - 1) / kKT);
     }
   } else {
     p.log2_group = 0;

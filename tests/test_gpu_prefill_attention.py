@@ -250,3 +250,36 @@ def test_prefill_api_validation(native_ops, device):
     bad[0, 0] = kc.shape[0] + 3
     with pytest.raises(IndexError, match="outside the cache"):
         kv_cache.paged_attention(q, kc, vc, bad.to(device), [100], scale=0.0625, query_lens=[10])
+
+
+def test_prefill_of_short_requests_in_a_padded_query_buffer(native_ops, device):
+    """A caller with static shapes passes a buffer of batch * max_query_len rows
+    whatever the requests hold: the same rows as without the padding, and the keys
+    split over the CUs all the same (about equal times; unsplit it takes 30x)."""
+    lens, qlens, bs = [16384], [8], 128
+    kc, vc, table = build_cache(device, lens, 4, 256, bs, 3)
+    q = randn((512, 16, 256), 4, 1.0, torch.bfloat16)
+    run = [lambda n=n: _run_op(device, q[:n], kc, vc, table, lens, qlens, 1 / 16, True, max_query_len=512)
+           for n in (8, 512)]
+    exact, padded = (f() for f in run)
+    # Other splits of the keys round the softmax weights to bf16 against another
+    # maximum: independent errors of at most 2^-9, rms 2^-9 / sqrt(3), per weight and
+    # so in the rms of the outputs, on both sides, and as much again for the outputs'
+    # own rounding: 2.3e-3 of the norm expected, three times that allowed.
+    assert float((padded[:8].double() - exact.double()).norm() / exact.double().norm()) < 7e-3
+    loc = torch.tensor([0, 8], dtype=torch.int32, device=device)
+    args = (kc, vc, table.to(device), loc, torch.tensor(lens, dtype=torch.int32, device=device), 1 / 16, 512, 16384)
+    times = []
+    for n in (8, 512):
+        qd = q[:n].to(device)
+        event = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = math.inf
+        for _ in range(5):
+            event[0].record()
+            for _ in range(4):
+                torch.ops.vllm_ascend_hif8.hif8_paged_prefill_attention(qd, *args, True)
+            event[1].record()
+            event[1].synchronize()
+            best = min(best, event[0].elapsed_time(event[1]))
+        times.append(best)
+    assert times[1] < 5 * times[0], times
