@@ -499,11 +499,23 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_kernel(
 // What bounds it now is LDS: per step of a 256 x 128 block 1024 clocks of
 // fragment reads, ~500 of lookups and ~500 of copies and stores.
 //
-// kStages K steps of both tiles sit in LDS: three where they fit beside the
-// table and the code ring, so that a copy has two steps to land in, else two.
-constexpr int dma_stages(int bm, int bn, bool wdec) {
-  return 3 * (bm + bn) * kBK * 2 + (wdec ? 3 * bn * kBK : 0) + 512 <= 160 * 1024 ? 3 : 2;
+// kStages K steps of both tiles sit in LDS: three, so that a copy has two steps to
+// land in, where they fit beside the table and the code ring and leave a CU as many
+// blocks as two stages do, else two.  128 x 128 blocks keep two: with three (96 KiB)
+// one block instead of two fits a CU (MI355X, decoded weights, two against three
+// stages: 3000 x 2048 x 2048 37 against 46 us, 512 x 4096 x 4096 38.5 against 42.6).
+constexpr int dma_lds_bytes(int bm, int bn, bool wdec, int stages) {
+  return stages * (bm + bn) * kBK * 2 + (wdec ? 3 * bn * kBK : 0) + 512;
 }
+constexpr int dma_stages(int bm, int bn, bool wdec) {
+  constexpr int kLds = 160 * 1024;
+  const int three = kLds / dma_lds_bytes(bm, bn, wdec, 3);
+  return three > 0 && three == kLds / dma_lds_bytes(bm, bn, wdec, 2) ? 3 : 2;
+}
+static_assert(dma_stages(128, 128, false) == 2 && dma_stages(256, 128, false) == 3 &&
+                  dma_stages(256, 192, false) == 2 && dma_stages(256, 256, false) == 2 &&
+                  dma_stages(256, 128, true) == 2 && dma_stages(256, 192, true) == 2,
+              "two 128 x 128 blocks per CU; a third stage only where it costs no block");
 
 template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec>
 __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
