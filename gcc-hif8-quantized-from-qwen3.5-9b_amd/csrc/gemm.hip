@@ -1087,14 +1087,58 @@ int launch_prepared(const LinearArgs &a, const GemmPlan &p, uint8_t *ws) {
   return launch_plan<true>(a, p, abf, splits, partial);
 }
 
-// Whether a call runs gemm_skinny_kernel: every K that the tiles do not take,
-// up to 64 rows (one row tile reads the weight once), and more rows while the
-// 64 x 32 blocks still fit the CUs in one round and K is short.  MI355X, whole
-// call against the 128 x 128 tiles: M = 64 24576 x 4096 44.6 vs 54.5 us, 4096
-// x 4096 15.4 vs 25.3; M = 128 4096 x 4096 18.5 vs 28.6; M = 256 2048 x 4096
-// 18.1 vs 27.9; but M = 128 4096 x 12288 43 vs 37.7 and 24576 x 4096 70 vs 59.
+int launch_simple(const LinearArgs &a) {
+  const dim3 grid(unsigned((a.n + 255) / 256), unsigned(a.m));
+  gemm_simple_kernel<<<grid, 256, 0, a.stream>>>(static_cast<const uint8_t *>(a.act), a.act_scale, a.weight,
+                                                 a.channel_scale, a.bias, a.bias_dtype, a.out, a.out_dtype, int(a.m),
+                                                 int(a.n), int(a.k));
+  return check_launch("soft_hif8 GEMM (generic)");
+}
+
+// Whether a call of more than four rows runs gemm_skinny_kernel: every K that the
+// tiles do not take, up to 64 rows (one row tile reads the weight once), and more
+// rows while the 64 x 32 blocks still fit the CUs in one round.  MI355X, whole call
+// against the tiles: M = 64 24576 x 4096 44.6 vs 54.5 us, 4096 x 4096 15.4 vs 25.3; M
+// = 128 4096 x 4096 18.5 vs 28.6; M = 256 2048 x 4096 18.1 vs 27.9; but M = 128 4096 x
+// 12288 43 vs 37.7 and 24576 x 4096 70 vs 59.  The lines between:
+//   * above 64 rows a block walks the whole K for its rows alone: M K up to 10
+//     million (1280 x 256 x 8192 34.6 vs 32.6, 2048 x 256 x 4096 29.6 vs 30.4, 2500 x
+//     128 x 4096 33.3 vs 31.7, 2048 x 128 x 8192 49 vs 32), or K <= 3072 (4096 x 128
+//     32.9 vs 36.5), up to 4096 rows (6000 x 64 x 512 17.4 vs 15.1);
+//   * above 48 rows the 128-tiles of N >= 57344 fill the chip (M = 64 N = 49152 K =
+//     1024 29.6 vs 29.9, 57344 34.5 vs 30.5, 151936 x 4096 235 vs 219);
+//   * long K, which no split shortens here, where the tiles' splits spread it (to 32
+//     steps a block, or over all CUs): 33 rows and more from K > 12288 on (M = 64 2048
+//     x 12288 26.9 vs 31.3, x 16384 40.6 vs 30.8), 17 to 32 rows over narrow N from
+//     16384 (M = 32 2048 x 16384 29.1 vs 28.8, x 20480 38.6 vs 33.3; 4096 x 20480 40.9
+//     vs 43.1), fewer from 32768 (M = 16 512 x 32768 27.5 vs 32, x 65536 67 vs 44).
 bool skinny_rule(int64_t m, int64_t n, int64_t k) {
-  return k % kBK != 0 || m <= 64 || (k <= 8192 && (n + 31) / 32 * ((m + 63) / 64) <= 256);
+  if (k % kBK) return true;
+  if (m > 64)
+    return m <= 4096 && k <= 8192 && (k <= 3072 || m * k <= 10000000) && (n + 31) / 32 * ((m + 63) / 64) <= 256;
+  const int64_t limit = m <= 16 ? 32768 : m <= 32 ? 16384 : 12288;
+  if (!(m > 48 && n >= 57344) && !(k > limit && (m > 32 || n < 4096))) return true;
+  const GemmPlan p = plan_gemm(m, n, k);
+  const int64_t tiles = ((m + p.tile - 1) / p.tile) * ((n + p.bn - 1) / p.bn);
+  return tiles * p.splits < 256 && k / p.splits > 2048;
+}
+
+// Ragged K of so few products that gemm_simple_kernel alone (one output per thread,
+// 2048 wavefronts at a time) ends before two launches would.  MI355X, M = 64 N =
+// 1000: K = 17 4.6 vs 7.9 us, 33 6.7 vs 8.1, 45 8.0 vs 8.1; 128 x 4096 x 17 12.8 vs
+// 9.7; 2048 x 16384 x 1 53 vs 108; quantised in the call, K = 33 9.5 vs 9.6.
+bool simple_rule(int64_t m, int64_t n, int64_t k) {
+  return k % kBK && m <= 65535 && (k <= 2 || k * ((m * ((n + 63) / 64) + 2047) / 2048) < 33);
+}
+
+// One to four rows of a K the GEMV cannot stream in 16-byte chunks: whether the
+// few-row GEMM's two launches beat one output per wavefront, whose time goes with M, K
+// and, past some 3072 outputs, N.  MI355X: codes 1 x 1000 x 1037 8.5 vs 8.3 us, 4 x
+// 1000 x 333 8.5 vs 7.5, 4 x 4096 x 333 8.5 vs 9.7; quantised in the call 1 x 1000 x
+// 333 9.7 vs 7.5, x 1037 10 vs 15.6, 4 x 1000 x 333 9.8 vs 11.3, 2 x 65536 x 17 20.4
+// vs 27.7.  One line between the two, so that their outputs stay equal bit for bit.
+bool few_rows_rule(int64_t m, int64_t n, int64_t k) {
+  return k % 16 && (n >= 65536 || (m + 1) * k * std::max<int64_t>(n, 3072) >= int64_t(1400) * 3072);
 }
 
 }  // namespace
@@ -1109,30 +1153,23 @@ size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k) {
 
 size_t gemm_scratch_size(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > 0x7FFFFFFFll || n <= 0 || k <= 0) return 0;
-  // The GEMV streams rows of whole 16-byte chunks; other K leave it one output
-  // per wavefront (MI355X, a scheme call in a graph, 4 x 2900 x 4100 97.4 ->
-  // 17.3 us, 1 x 1000 x 2052 31.6 -> 14.6, 1 x 60 x 100 16.8 -> 13.8).
-  if (m <= 4 && k % 16 == 0) return 0;
-  return k % kBK ? skinny_workspace_size(m, k) : gemm_workspace_size(m, n, k);
+  if (m <= 4) return few_rows_rule(m, n, k) ? skinny_workspace_size(m, k) : 0;
+  if (simple_rule(m, n, k)) return 0;
+  // The fragments also where operands that are not 16-byte aligned keep the tiles away.
+  return std::max(skinny_workspace_size(m, k), gemm_workspace_size(m, n, k));
 }
 
 int launch_gemm(const LinearArgs &a) {
   if (a.act_kind != kActCodes)
     return fail(HIF8_ERR_UNSUPPORTED, "soft_hif8 GEMM takes uint8 activation codes");
   const bool tiled = a.k % kBK == 0 && aligned(a.act, 16) && aligned(a.weight, 16);
-  if (skinny_rule(a.m, a.n, a.k) && a.workspace && a.workspace_bytes >= skinny_workspace_size(a.m, a.k) &&
-      aligned(a.workspace, 256)) {
+  if ((!tiled || skinny_rule(a.m, a.n, a.k)) && !simple_rule(a.m, a.n, a.k) && a.workspace &&
+      a.workspace_bytes >= skinny_workspace_size(a.m, a.k) && aligned(a.workspace, 256)) {
     uint16_t *act = static_cast<uint16_t *>(a.workspace);
     const int st = launch_decode_fragments(a, act);
     return st ? st : launch_gemm_skinny(a, act);
   }
-  if (!tiled) {
-    const dim3 grid(unsigned((a.n + 255) / 256), unsigned(a.m));
-    gemm_simple_kernel<<<grid, 256, 0, a.stream>>>(
-        static_cast<const uint8_t *>(a.act), a.act_scale, a.weight, a.channel_scale, a.bias,
-        a.bias_dtype, a.out, a.out_dtype, int(a.m), int(a.n), int(a.k));
-    return check_launch("soft_hif8 GEMM (generic)");
-  }
+  if (!tiled) return launch_simple(a);
   const GemmPlan p = plan_gemm(a.m, a.n, a.k);
   const bool use_ws = a.workspace && a.workspace_bytes >= p.a_bytes + p.w_bytes + p.part_bytes &&
                       aligned(a.workspace, 256);
@@ -1155,20 +1192,29 @@ size_t gemm_static_workspace_size(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || m > 0x7FFFFFFFll || n > 0x7FFFFFFFll || k > 0x7FFFFFFFll || n <= 0 || k <= 0) return 0;
   if (m <= 4 && k % 16 == 0) return 0;  // the GEMV's
   const size_t scales = (size_t(m) * sizeof(float) + 255) / 256 * 256;
-  // Fragments also where a weight that is not 16-byte aligned keeps the tiles away.
-  return scales + std::max(skinny_workspace_size(m, k), k % kBK ? 0 : gemm_workspace_size(m, n, k));
+  return scales + std::max(skinny_workspace_size(m, k), gemm_workspace_size(m, n, k));
 }
 
 int launch_gemm_static(const LinearArgs &a) {
+  const bool few = a.m <= 4 && !few_rows_rule(a.m, a.n, a.k);
+  // One row is faster quantised in every block of the GEMV than by a launch before it.
+  if (few && a.m == 1) return launch_gemv(a);
   float *row_scale = static_cast<float *>(a.workspace);
   uint8_t *ws = static_cast<uint8_t *>(a.workspace) + (size_t(a.m) * sizeof(float) + 255) / 256 * 256;
   uint16_t *act = reinterpret_cast<uint16_t *>(ws);
+  LinearArgs b = a;
+  b.act_scale = row_scale;
+  if (few || (a.m > 4 && simple_rule(a.m, a.n, a.k))) {
+    b.act = ws;
+    b.act_kind = kActCodes;
+    const int st = hif8_static_quant(a.act, a.act_kind == kActBf16 ? HIF8_DTYPE_BF16 : HIF8_DTYPE_FP16, a.m, a.k,
+                                     a.act_scale, 1, ws, row_scale, reinterpret_cast<hif8_stream_t>(a.stream));
+    return st ? st : few ? launch_gemv(b) : launch_simple(b);
+  }
   const bool fragments = skinny_rule(a.m, a.n, a.k) || !aligned(a.act, 16) || !aligned(a.weight, 16);
   int st = launch_static_operand(a.act, a.act_kind == kActBf16, a.act_scale, act, row_scale, a.m, a.k, fragments,
                                  a.stream);
   if (st) return st;
-  LinearArgs b = a;
-  b.act_scale = row_scale;
   if (fragments) return launch_gemm_skinny(b, act);
   const GemmPlan p = plan_gemm(a.m, a.n, a.k);
   if (p.w_pre) {

@@ -150,7 +150,9 @@ size_t soft_hif8_gemm_workspace_size(int64_t m, int64_t n, int64_t k);
  * The workspace with which soft_hif8_gemm_with_workspace runs fastest: the size
  * above, and for K that is no multiple of 64 (16 for M <= 4), where that is 0 and
  * a call without workspace computes one output per thread or wavefront, the bf16
- * activation fragments with which the call runs on the matrix cores.
+ * activation fragments with which the call runs on the matrix cores (0 where the
+ * call is so small that it ends sooner without).  Never less than the fragments
+ * where it is not 0: operands that are not 16-byte aligned run on them at any K.
  */
 size_t soft_hif8_gemm_scratch_size(int64_t m, int64_t n, int64_t k);
 

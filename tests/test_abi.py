@@ -195,3 +195,40 @@ def test_qk_norm_rope_rejects_more_blocks_than_a_launch_holds(lib):
     for heads in (248, 1 << 20):
         assert f(*[_p(16)] * 6, 4, 16, *[_p(16)] * 4, 65536, heads, 4, 64, 64, 1e-6, None) == 1
         assert b"unsupported dimensions" in lib.hif8_last_error()
+
+
+def _scratch(lib, m, n, k, which="scratch"):
+    f = getattr(lib, f"soft_hif8_gemm_{which}_size")
+    f.argtypes, f.restype = [ctypes.c_int64] * 3, ctypes.c_size_t
+    return f(m, n, k)
+
+
+def _fragments(m, k):
+    return -(-m // 16) * 16 * (-(-k // 64) * 64) * 2
+
+
+@pytest.mark.parametrize("m,n,k,few", [
+    (64, 24576, 4096, True), (128, 4096, 4096, True), (256, 2048, 4096, True), (64, 2048, 12288, True),
+    # tall and narrow
+    (1280, 256, 4096, True), (2048, 128, 8192, False), (2500, 64, 4096, False), (4096, 128, 3072, True),
+    (8192, 64, 512, False),
+    # wide enough for the tiles
+    (60, 49152, 1024, True), (60, 65536, 1024, False), (40, 65536, 1024, True),
+    # long K: split over blocks by the tiles, unless its steps do not divide
+    (64, 512, 16384, False), (64, 512, 64 * 257, True), (24, 2048, 20480, False), (24, 4096, 20480, True),
+    (16, 512, 32768, True), (16, 512, 65536, False),
+])
+def test_workspace_size_tells_the_kernel_of_whole_steps(lib, m, n, k, few):
+    """Where the few-row GEMM is the faster one its fragments are the workspace, elsewhere
+    the tiles' plan; the scratch always holds the fragments, for unaligned operands."""
+    assert (_scratch(lib, m, n, k, "workspace") == _fragments(m, k)) == few
+    assert _scratch(lib, m, n, k) == max(_scratch(lib, m, n, k, "workspace"), _fragments(m, k))
+
+
+@pytest.mark.parametrize("m,n,k,few", [
+    (5, 1000, 17, False), (64, 1000, 31, False), (64, 1000, 45, True), (128, 4096, 17, True), (2048, 16384, 1, False),
+    (77, 1000, 2052, True), (1, 8, 100, False), (1, 1000, 690, False), (1, 1000, 705, True), (4, 1000, 100, False), (4, 1000, 333, True),
+    (1, 30000, 100, True), (2, 4096, 100, False), (3, 1000, 1040, False),
+])
+def test_scratch_size_is_zero_where_a_ragged_call_ends_sooner_without(lib, m, n, k, few):
+    assert _scratch(lib, m, n, k) == (_fragments(m, k) if few else 0)

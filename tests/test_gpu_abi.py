@@ -110,3 +110,49 @@ def test_static_fused_gemm_abi_equals_quant_then_gemm(lib, device, m, n, k, xdty
                                            m, n, k, None) == 0, lib.hif8_last_error()
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# Rows of the tiles (unaligned: fragments instead), of the few-row GEMM, of one to four
+# rows with and without it, and of a ragged call of few products.
+@pytest.mark.parametrize("m,n,k", [(300, 1000, 256), (130, 72, 8256), (20, 40, 128), (4, 100, 300), (3, 40, 100),
+                                   (1, 40, 690), (5, 40, 17)])
+@pytest.mark.parametrize("off_x,off_w", [(1, 0), (0, 1), (3, 5)])
+def test_operands_that_are_not_16_byte_aligned(lib, device, m, n, k, off_x, off_w):
+    """hif8_static_linear and soft_hif8_gemm_with_workspace (scratch size) on operands
+    that start off_x elements and off_w bytes into their buffers: equal to each other
+    bit for bit, and to the oracle."""
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+    for f in (lib.soft_hif8_gemm_scratch_size, lib.hif8_static_linear_workspace_size):
+        f.argtypes, f.restype = [i64] * 3, ctypes.c_size_t
+    lib.hif8_static_quant.argtypes = [ptr, ctypes.c_int, i64, i64, ptr, i64, ptr, ptr, ptr]
+    lib.hif8_static_linear.argtypes = [ptr, ctypes.c_int] + [ptr] * 4 + [ctypes.c_int, ptr, ctypes.c_int] + \
+        [i64] * 3 + [ptr, ctypes.c_size_t, ptr]
+    g = torch.Generator().manual_seed(m + n + k)
+
+    def shifted(t, off):
+        buf = torch.zeros(t.numel() + 16, dtype=t.dtype, device=device)
+        buf[off:off + t.numel()] = t.reshape(-1).to(device)
+        return buf[off:off + t.numel()].view(t.shape)
+
+    x = shifted((torch.randn(m, k, generator=g) * 3).to(torch.bfloat16), off_x)
+    w_np = random_codes((n, k), seed=n + k)
+    w = shifted(torch.from_numpy(w_np), off_w)
+    fixed = torch.tensor([0.0009765625 * 1.1], device=device)
+    cs = (torch.rand(n, generator=g) + 0.5).to(device)
+    codes = shifted(torch.zeros(m, k, dtype=torch.uint8), off_x)
+    rs = torch.empty(m, dtype=torch.float32, device=device)
+    out = [torch.empty(m, n, dtype=torch.bfloat16, device=device) for _ in range(2)]
+    sizes = [lib.soft_hif8_gemm_scratch_size(m, n, k), lib.hif8_static_linear_workspace_size(m, n, k)]
+    ws = [torch.empty(max(s, 1), dtype=torch.uint8, device=device) for s in sizes]
+    torch.cuda.synchronize()
+    assert lib.hif8_static_quant(_ptr(x), BF16, m, k, _ptr(fixed), 1, _ptr(codes), _ptr(rs), None) == 0
+    assert lib.soft_hif8_gemm_with_workspace(
+        _ptr(codes), _ptr(w), _ptr(rs), _ptr(cs), None, -1, _ptr(out[0]), BF16, m, n, k,
+        _ptr(ws[0]) if sizes[0] else None, sizes[0], None) == 0, lib.hif8_last_error()
+    assert lib.hif8_static_linear(_ptr(x), BF16, _ptr(w), _ptr(fixed), _ptr(cs), None, -1, _ptr(out[1]), BF16, m, n,
+                                  k, _ptr(ws[1]), sizes[1], None) == 0, lib.hif8_last_error()
+    torch.cuda.synchronize()
+    want = o.linear_u8_u8(codes.cpu().numpy(), rs.cpu().numpy(), w_np, cs.cpu().numpy(), None)
+    torch.testing.assert_close(out[0].cpu().float(), torch.from_numpy(want.astype(np.float32)), rtol=1e-2, atol=1e-2,
+                               equal_nan=True)
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))

@@ -118,6 +118,9 @@ def test_gemm_shapes_and_tails(native_ops, device, rows, channels, k):
     # wavefronts, odd rows; M and N: edges of the 16-row tiles and of a 64-row tile.
     (5, 1, 64), (16, 15, 63), (17, 33, 65), (64, 16, 1024), (65, 40, 130), (48, 100, 1089), (130, 18, 100),
     (20, 4200, 192), (70, 2100, 333), (256, 64, 448),
+    # sizes at which another kernel is the faster one: tall, long K, few products
+    (4096, 33, 192), (2500, 20, 4096), (1250, 70, 8192), (40, 130, 16384), (20, 70, 20480), (64, 57344, 64),
+    (5, 100, 31), (130, 1000, 17), (3, 1000, 100), (1, 40, 690),
 ])
 def test_few_row_and_ragged_gemm(native_ops, device, rows, channels, k):
     """The streaming GEMM (up to 64 rows, or any K): values against the float64
@@ -154,7 +157,7 @@ def test_few_row_gemm_of_rows_beyond_32_bit_offsets(native_ops, device, rows, k)
     _check(y, o.linear_u8_u8(codes, ts, weights, cs, None))
 
 
-@pytest.mark.parametrize("rows,channels,k", [(5, 2 ** 28 + 2 ** 20 + 17, 3), (2 ** 27 + 2 ** 20 + 5, 3, 1)])
+@pytest.mark.parametrize("rows,channels,k", [(5, 2 ** 28 + 2 ** 20 + 17, 3), (2 ** 27 + 2 ** 20 + 5, 3, 3)])
 def test_few_row_gemm_of_more_tiles_than_one_launch_holds(native_ops, device, rows, channels, k):
     """More weight rows, or activation rows, than the threads of one launch (2^32)
     cover: every output against a float32 product, which is exact for these codes."""
@@ -193,7 +196,9 @@ def test_weight_decoding_tiles_of_few_steps(native_ops, device, rows, channels, 
     (5, 40, 64), (17, 33, 100), (64, 4200, 1040), (70, 2100, 333), (129, 136, 12288), (300, 1000, 2048),
     (512, 2048, 4096), (2048, 256, 1024),
     # rows of a decode step whose K is no multiple of 16
-    (3, 40, 100), (4, 4200, 1037),
+    (3, 40, 100), (4, 4200, 1037), (4, 100, 260), (4, 100, 300),
+    # few products; tall; long K
+    (5, 40, 17), (64, 1000, 31), (300, 40, 17), (2500, 70, 4096), (33, 130, 16384),
 ])
 def test_static_linear_equals_quant_then_gemm(native_ops, device, rows, channels, k, xdtype):
     from hif8_rocm import native
