@@ -501,9 +501,11 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_kernel(
 //
 // kStages K steps of both tiles sit in LDS: three, so that a copy has two steps to
 // land in, where they fit beside the table and the code ring and leave a CU as many
-// blocks as two stages do, else two.  128 x 128 blocks keep two: with three (96 KiB)
-// one block instead of two fits a CU (MI355X, decoded weights, two against three
-// stages: 3000 x 2048 x 2048 37 against 46 us, 512 x 4096 x 4096 38.5 against 42.6).
+// blocks as two stages do, else two.  128 x 128 blocks (two per CU with 64 KiB, one
+// with 96) take three while the grid has no more than one block per CU: MI355X,
+// decoded weights, two against three stages, 128 x 4096 x 4096 (256 blocks) 26.2
+// against 22.3 us, 512 x 1024 x 4096 24.6 against 21.8, but 3000 x 2048 x 2048 (384)
+// 37 against 46, 512 x 4096 x 4096 (512) 38.5 against 42.6.
 constexpr int dma_lds_bytes(int bm, int bn, bool wdec, int stages) {
   return stages * (bm + bn) * kBK * 2 + (wdec ? 3 * bn * kBK : 0) + 512;
 }
@@ -517,7 +519,7 @@ static_assert(dma_stages(128, 128, false) == 2 && dma_stages(256, 128, false) ==
                   dma_stages(256, 128, true) == 2 && dma_stages(256, 192, true) == 2,
               "two 128 x 128 blocks per CU; a third stage only where it costs no block");
 
-template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec>
+template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec, int kStages>
 __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
     const uint16_t *__restrict__ A, const float *__restrict__ ts, const void *__restrict__ Wv,
     const float *__restrict__ cs, const void *__restrict__ bias, int bias_dtype,
@@ -532,7 +534,6 @@ __global__ __launch_bounds__(kWave * kWavesM * kWavesN, 1) void gemm_dma_kernel(
   static_assert(kDmaA * kWaves * 1024 == int(kStageA) && (kWDec || kDmaB * kWaves * 1024 == int(kStageB)),
                 "tile copies split evenly over the waves");
   constexpr int kDec = kWDec ? kBN * kBK / 8 / kT : 0;  // 8-code W chunks per thread and step
-  constexpr int kStages = dma_stages(kBM, kBN, kWDec);
   // 1 KiB copies of a code tile (16 rows of 64 codes each) and their number per
   // wave; the last ones repeat where they do not divide over the waves.
   constexpr int kCodeCopies = kBN * kBK / 1024, kDmaC = kWDec ? (kCodeCopies + kWaves - 1) / kWaves : 0;
@@ -1022,20 +1023,20 @@ int launch_tiled(const LinearArgs &a, const void *act, const void *wt, int split
 
 // Launch of gemm_dma_kernel (+ the split-K reduce when partial is set); wt
 // is the bf16 weight, or (kWDec) the codes.
-template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec = false>
+template <int kBM, int kBN, int kWavesM, int kWavesN, bool kWDec = false, int kStages = dma_stages(kBM, kBN, kWDec)>
 int launch_dma(const LinearArgs &a, const uint16_t *act, const void *wt, int splits, float *partial) {
-  constexpr size_t kSmem = std::max<size_t>(dma_stages(kBM, kBN, kWDec) * size_t(kBM + kBN) * kBK * 2 +
+  constexpr size_t kSmem = std::max<size_t>(kStages * size_t(kBM + kBN) * kBK * 2 +
                                                 (kWDec ? 3 * size_t(kBN) * kBK : 0),
                                             size_t(kWavesM * kWavesN) *
                                                 epilogue_region_bytes<kBM / kWavesM / 16, kBN / kWavesN / 16>());
   constexpr int kT = kWave * kWavesM * kWavesN;
   if (const int st = reserve_dynamic_lds(
-          reinterpret_cast<const void *>(&gemm_dma_kernel<kBM, kBN, kWavesM, kWavesN, kWDec>), kSmem,
+          reinterpret_cast<const void *>(&gemm_dma_kernel<kBM, kBN, kWavesM, kWavesN, kWDec, kStages>), kSmem,
           "soft_hif8 GEMM"))
     return st;
   const int64_t tiles = ((a.n + kBN - 1) / kBN) * ((a.m + kBM - 1) / kBM);
   const dim3 grid(unsigned((tiles * splits + 7) / 8 * 8));
-  gemm_dma_kernel<kBM, kBN, kWavesM, kWavesN, kWDec><<<grid, kT, kSmem, a.stream>>>(
+  gemm_dma_kernel<kBM, kBN, kWavesM, kWavesN, kWDec, kStages><<<grid, kT, kSmem, a.stream>>>(
       act, a.act_scale, wt, a.channel_scale, a.bias, a.bias_dtype, a.out, a.out_dtype, int(a.m), int(a.n),
       int(a.k), partial, splits, int(a.k / kBK / splits));
   int st = check_launch("soft_hif8 GEMM");
@@ -1051,6 +1052,8 @@ int launch_bf16_operands(const LinearArgs &a, const GemmPlan &p, const uint16_t 
   if (p.tile == 256 && p.bn == 192) return launch_dma<256, 192, 4, 2>(a, act, wt, splits, partial);
   if (p.tile == 256 && p.bn == 128) return launch_dma<256, 128, 4, 2>(a, act, wt, splits, partial);
   if (p.tile == 256) return launch_dma<256, 256, 4, 2>(a, act, wt, splits, partial);
+  if (((a.m + 127) / 128) * ((a.n + 127) / 128) * splits <= 256)
+    return launch_dma<128, 128, 2, 2, false, 3>(a, act, wt, splits, partial);
   return launch_dma<128, 128, 2, 2>(a, act, wt, splits, partial);
 }
 
