@@ -271,11 +271,16 @@ class HybridModel:
         # Decode quantizes projection inputs inside the glue kernels; False
         # runs the scheme's own quant per projection (same codes, more launches).
         self.fuse_input_quant = True
-        # Prefill runs the delta rule in torch; True takes the HIP kernels of
-        # gated_delta_chunked (1.6 ms less per linear-attention layer of a
-        # 512-token prompt).  They are nearer to float64, but another FP32
-        # rounding, which changes single HiF8 codes downstream: off by
-        # default, so that a model's prefill repeats its results bit for bit.
+        # Prefill runs the delta rule in torch; True takes gated_delta_chunked, whose
+        # HIP kernels spend 1.6 ms less per linear-attention layer of a 512-token
+        # prompt, repeat themselves bit for bit and are nearer to float64.  Off by
+        # default because they round FP32 differently and static HiF8 quant of
+        # random-init weights amplifies that over 32 layers (amax -> 32768): the
+        # cosine of decode against prefill logits averages 0.73 over twelve prompts
+        # with either form (torch 0.60 .. 0.81, kernels 0.66 .. 0.78) but moves by up
+        # to 0.17 on one, and the prompt on which the full-size test holds decode to
+        # the chunked prefill's cosine less 0.05 meets that with the torch form (0.768
+        # against 0.750) and not with the kernels (0.755 against 0.808).
         self.delta_kernel = False
         # Decode runs the linear-attention mixer as the conv-epilogue qkvz GEMV
         # + one block per value head where the shapes allow; False keeps the

@@ -530,3 +530,40 @@ def test_qk_norm_rope_cache_equals_rope_then_cache_write(native_ops, device, d, 
     assert torch.equal(got, q)
     assert torch.equal(caches[2], caches[0]) and torch.equal(caches[3], caches[1])
     assert int((caches[2] != 0).any(-1).sum()) == 2 * hkv
+
+
+def test_model_prefill_on_the_delta_kernels(native_ops, device, monkeypatch):
+    """model.delta_kernel, a prefill in two chunks: every linear-attention layer hands gated_delta_chunked
+    a call its kernels take, whose outputs and state match the float64 recurrence; a
+    second run repeats logits and states bit for bit."""
+    from hif8_rocm import synthetic_model
+    from hif8_rocm.synthetic_model import HybridConfig, HybridModel
+
+    model = HybridModel(HybridConfig(**dict(TINY, layers=2, lin_k_dim=64)), device, seed=5)
+    model.calibrate(batch=1, tokens=32)
+    assert not model.delta_kernel
+    model.delta_kernel = True
+    b, t, more = 2, 70, 9
+    ids = torch.randint(0, model.cfg.vocab, (b, t + more), generator=torch.Generator().manual_seed(2)).to(device)
+    calls, inner = [], synthetic_model.gated_delta_chunked
+
+    def recorded(q, k, v, g, beta, state):
+        assert synthetic_model._delta_kernel_takes(q, k, v, g, beta, state, 64)
+        want_state = state.double()
+        want = torch.stack([synthetic_model.gated_delta_step(want_state, *(x[:, :, i].double() for x in (q, k, v, g, beta)))
+                            for i in range(q.shape[2])], dim=2)
+        out = inner(q, k, v, g, beta, state)
+        calls.append(max(float((x.double() - y).norm() / y.norm()) for x, y in ((out, want), (state, want_state))))
+        return out
+
+    monkeypatch.setattr(synthetic_model, "gated_delta_chunked", recorded)
+    runs = []
+    for _ in range(2):
+        st = model.new_state(b, t + more)
+        for first, n in ((0, t), (t, more)):
+            pos = torch.arange(first, first + n, device=device).expand(b, n).contiguous()
+            st.seq_lens.fill_(first + n)
+            logits = model.forward(st, ids[:, first:first + n].contiguous(), pos, decode=False)
+        runs.append([logits, *st.rec_states])
+    assert len(calls) == 2 * 2 * 2 and max(calls) < 1e-6, calls  # two layers, chunks and runs
+    assert all(torch.equal(x, y) for x, y in zip(*runs))
