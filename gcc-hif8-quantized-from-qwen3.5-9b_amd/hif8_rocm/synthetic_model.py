@@ -457,7 +457,8 @@ class HybridModel:
         gdecay = -torch.exp(L["A_log"]) * torch.nn.functional.softplus(ba[..., c.lin_v_heads:] + L["dt_bias"])
         # Causal depthwise conv over time with the carried state (width conv_kernel).
         conv_state = st.conv_states[idx]
-        if self._prefill_kernels(b, t):
+        glue = not decode and self._prefill_kernels(b, t)  # a decode step stays in torch throughout
+        if glue:
             mixed = torch.ops.vllm_ascend_hif8.hif8_conv_tokens(qkvz, L["conv"], conv_state)
         else:
             seq = torch.cat([conv_state, mixed.transpose(1, 2)], dim=-1)       # [B, C, K-1+T]
@@ -479,7 +480,7 @@ class HybridModel:
             rule = gated_delta_chunked if self.delta_kernel else _gated_delta_torch
             o = rule(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2),
                      gdecay.transpose(1, 2), beta.transpose(1, 2), state).transpose(1, 2)
-        if self._prefill_kernels(b, t):
+        if glue:
             o = torch.ops.vllm_ascend_hif8.hif8_gated_rms_norm(o, qkvz, 2 * c.lin_qk_width + c.lin_v_width,
                                                                L["out_norm"], c.rms_eps)
             return L["out"](o.reshape(b * t, c.lin_v_width)).reshape(b, t, -1)

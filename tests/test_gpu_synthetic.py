@@ -567,3 +567,29 @@ def test_model_prefill_on_the_delta_kernels(native_ops, device, monkeypatch):
         runs.append([logits, *st.rec_states])
     assert len(calls) == 2 * 2 * 2 and max(calls) < 1e-6, calls  # two layers, chunks and runs
     assert all(torch.equal(x, y) for x, y in zip(*runs))
+
+
+def test_torch_decode_steps_run_no_glue_kernel(model, device):
+    """The torch decode steps that the fused ones are tested against call no glue
+    kernel of this library, so that they do not share a mistake with them."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Record(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.ops = set()
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops.add(func._schema.name)
+            return func(*args, **(kwargs or {}))
+
+    c, b = model.cfg, 2
+    st = model.new_state(b, 8)
+    st.seq_lens.fill_(1)
+    x = torch.randn(b, 1, c.hidden, device=device).to(torch.bfloat16)
+    with Record() as seen:
+        model._linear_attention(model.layers[0], 0, st, x, decode=True)
+        model._attention(model.layers[3], 0, st, x, torch.zeros(b, 1, dtype=torch.int64, device=device), True)
+    own = {name.split("::")[1] for name in seen.ops if name.startswith("vllm_ascend_hif8::")}
+    assert own <= {"hif8_static_quant", "soft_hif8_gemv", "soft_hif8_gemm", "soft_hif8_static_fused_gemm",
+                   "hif8_static_linear", "hif8_kv_cache_write", "hif8_paged_decode_attention"}, own
