@@ -883,7 +883,8 @@ extern "C" int hif8_qk_norm_rope(const uint16_t *qkv, const uint16_t *q_norm, co
                                  int64_t num_kv_heads, int64_t head_size, int64_t rotary_dim, float eps,
                                  hif8_stream_t stream) {
   clear_error();
-  if (!qkv || !q_norm || !k_norm || !pos || !inv_freq || !q_out || !k_out || !v_out || (slots && !block_table))
+  if (!qkv || !q_norm || !k_norm || !pos || !inv_freq || !q_out || !k_out || !v_out ||
+      (slots && !block_table && max_blocks > 0))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope: null pointer argument");
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||
       rotary_dim < 0 || rotary_dim > head_size || rotary_dim % 2 || block_size <= 0 || batch > 65536 ||

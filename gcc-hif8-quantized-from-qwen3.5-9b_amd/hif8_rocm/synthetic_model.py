@@ -408,10 +408,10 @@ class HybridModel:
         qkv = L["qkv"](h.reshape(b * t, -1)).reshape(b, t, -1)
         if not decode and self._rope_kernel(b * t):
             # Row i of the fused kernel is one token: norms, rotary and the split
-            # in one launch (its cache slots are not used: _slots below checks them).
+            # in one launch (a table of no columns: _slots below makes the slots).
             q, k, v, _ = torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope(
                 qkv.reshape(b * t, -1), L["q_norm"], L["k_norm"], pos.reshape(b * t).to(torch.int64), self.inv_freq,
-                st.block_table[:b].repeat_interleave(t, dim=0), c.block_size, c.heads, c.kv_heads, c.head_dim,
+                st.block_table.new_empty((b * t, 0)), c.block_size, c.heads, c.kv_heads, c.head_dim,
                 c.rms_eps)
             q, k, v = (x.reshape(b, t, -1, c.head_dim) for x in (q, k, v))
         else:

@@ -474,6 +474,10 @@ int hif8_gdn_decode_head_quant(const float *conv, const uint16_t *mixed_qkvz, in
                                float *rec_state, const uint16_t *out_norm, const float *input_scale, uint8_t *codes,
                                float *row_scale, int64_t batch, int64_t k_heads, int64_t v_heads, int64_t k_dim,
                                int64_t v_dim, float eps, hif8_stream_t stream);
+/* RMS norm and rotary of the q and k heads of qkv [batch, num_heads + 2 num_kv_heads,
+ * head_size], v copied, and (slots not null) the cache slot of each row's position:
+ * block_table [batch, max_blocks]; a position outside it, or any with max_blocks 0
+ * (no table), gets -1.  head_size <= 256. */
 int hif8_qk_norm_rope(const uint16_t *qkv, const uint16_t *q_norm, const uint16_t *k_norm, const int64_t *pos,
                       const float *inv_freq, const int32_t *block_table, int64_t max_blocks, int64_t block_size,
                       uint16_t *q_out, uint16_t *k_out, uint16_t *v_out, int64_t *slots, int64_t batch,

@@ -6,6 +6,7 @@ decoding token for token."""
 
 import pytest
 import torch
+import torch.utils._python_dispatch
 
 pytestmark = pytest.mark.gpu
 
@@ -569,20 +570,24 @@ def test_model_prefill_on_the_delta_kernels(native_ops, device, monkeypatch):
     assert all(torch.equal(x, y) for x, y in zip(*runs))
 
 
+class Record(torch.utils._python_dispatch.TorchDispatchMode):
+    """The operators called and the sizes of the int32 tensors they return."""
+
+    def __init__(self):
+        super().__init__()
+        self.ops, self.int32 = set(), [0]
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        out = func(*args, **(kwargs or {}))
+        self.ops.add(func._schema.name)
+        self.int32 += [t.numel() for t in (out if isinstance(out, (list, tuple)) else [out])
+                       if isinstance(t, torch.Tensor) and t.dtype == torch.int32]
+        return out
+
+
 def test_torch_decode_steps_run_no_glue_kernel(model, device):
     """The torch decode steps that the fused ones are tested against call no glue
     kernel of this library, so that they do not share a mistake with them."""
-    from torch.utils._python_dispatch import TorchDispatchMode
-
-    class Record(TorchDispatchMode):
-        def __init__(self):
-            super().__init__()
-            self.ops = set()
-
-        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
-            self.ops.add(func._schema.name)
-            return func(*args, **(kwargs or {}))
-
     c, b = model.cfg, 2
     st = model.new_state(b, 8)
     st.seq_lens.fill_(1)
@@ -593,3 +598,26 @@ def test_torch_decode_steps_run_no_glue_kernel(model, device):
     own = {name.split("::")[1] for name in seen.ops if name.startswith("vllm_ascend_hif8::")}
     assert own <= {"hif8_static_quant", "soft_hif8_gemv", "soft_hif8_gemm", "soft_hif8_static_fused_gemm",
                    "hif8_static_linear", "hif8_kv_cache_write", "hif8_paged_decode_attention"}, own
+
+
+def test_prefill_makes_no_table_per_token(model, device):
+    """The rotary kernel of a prefill gets no block table (a row of pages per token
+    would grow with the square of the prompt); without one its slots are -1 and the
+    heads the same."""
+    c, b, t = model.cfg, 2, 40
+    st = model.new_state(b, t)
+    st.seq_lens.fill_(t)
+    x = torch.randn(b, t, c.hidden, device=device).to(torch.bfloat16)
+    pos = torch.arange(t, device=device).expand(b, t).contiguous()
+    with Record() as seen:
+        model._attention(model.layers[3], 0, st, x, pos, False)
+    assert "vllm_ascend_hif8::hif8_qk_norm_rope" in seen.ops
+    assert max(seen.int32) <= st.block_table.numel()
+    L = model.layers[3]
+    qkv = L["qkv"](x.reshape(b * t, -1))
+    rows = st.block_table.repeat_interleave(t, dim=0)
+    args = (qkv, L["q_norm"], L["k_norm"], pos.reshape(-1), model.inv_freq)
+    sizes = (c.block_size, c.heads, c.kv_heads, c.head_dim, c.rms_eps)
+    want, got = (torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope(*args, table, *sizes) for table in (rows, rows[:, :0]))
+    assert all(torch.equal(p, q) for p, q in zip(got[:3], want[:3]))
+    assert torch.equal(want[3], model._slots(st, pos)) and bool((got[3] == -1).all())
