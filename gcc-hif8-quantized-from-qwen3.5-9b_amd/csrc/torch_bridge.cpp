@@ -985,6 +985,11 @@ std::tuple<at::Tensor, at::Tensor> Hif8GdnDecodeHeadQuantMeta(
           at::empty({conv.size(0)}, mixed.options().dtype(at::kFloat))};
 }
 
+// Marks a tensor as changed in place, as torch's own in-place operations do: autograd
+// then refuses a backward through an earlier value of it (and torch an inference
+// tensor outside inference mode).
+void MarkChanged(const at::Tensor &t) { t.unsafeGetTensorImpl()->bump_version(); }
+
 // The gated delta rule over many tokens: q, k [B, H, T, dk], v [B, H, T, dv], g,
 // beta [B, H, T] of any strides (copied where rows are not contiguous or q / k
 // rows not 16-byte aligned), state [B, H, dk, dv] contiguous, updated in place.
@@ -1005,6 +1010,7 @@ at::Tensor Hif8GatedDelta(const at::Tensor &q, const at::Tensor &k, const at::Te
   TORCH_CHECK(g.sizes() == v.sizes().slice(0, 3) && beta.sizes() == g.sizes(), "hif8_gated_delta: g / beta shape");
   TORCH_CHECK(state.size(0) == batch && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv,
               "hif8_gated_delta: state shape");
+  MarkChanged(state);
   const c10::OptionalDeviceGuard guard(state.device());
   auto rowwise = [](const at::Tensor &t, bool vec) {
     bool ok = t.stride(3) == 1;
@@ -1043,6 +1049,7 @@ at::Tensor Hif8ConvTokens(const at::Tensor &x, const at::Tensor &conv_weight, at
                   x.size(2) >= channels, "hif8_conv_tokens: conv_state [B, C, width - 1], x [B, T, >= C]");
   CheckSameDevice(conv_weight, x.device(), "conv_weight");
   CheckSameDevice(conv_state, x.device(), "conv_state");
+  MarkChanged(conv_state);
   const c10::OptionalDeviceGuard guard(x.device());
   auto out = at::empty({batch, tokens, channels}, x.options().dtype(at::kFloat));
   CheckStatus(hif8_conv_tokens(reinterpret_cast<const uint16_t *>(x.data_ptr()), x.size(2),
@@ -1079,7 +1086,8 @@ at::Tensor Hif8GatedRmsNorm(const at::Tensor &o, const at::Tensor &mixed, int64_
   return out;
 }
 
-at::Tensor Hif8ConvTokensMeta(const at::Tensor &x, const at::Tensor &conv_weight, at::Tensor &) {
+at::Tensor Hif8ConvTokensMeta(const at::Tensor &x, const at::Tensor &conv_weight, at::Tensor &conv_state) {
+  MarkChanged(conv_state);
   return at::empty({x.size(0), x.size(1), conv_weight.size(0)}, x.options().dtype(at::kFloat));
 }
 
@@ -1088,7 +1096,8 @@ at::Tensor Hif8GatedRmsNormMeta(const at::Tensor &o, const at::Tensor &mixed, in
 }
 
 at::Tensor Hif8GatedDeltaMeta(const at::Tensor &, const at::Tensor &, const at::Tensor &v, const at::Tensor &,
-                              const at::Tensor &, at::Tensor &) {
+                              const at::Tensor &, at::Tensor &state) {
+  MarkChanged(state);
   return at::empty(v.sizes(), v.options());
 }
 

@@ -64,6 +64,22 @@ def test_gated_delta_leaves_autograd_and_other_types_to_torch(native_ops, device
         assert takes(*tensors, state, 64)
 
 
+def test_gated_delta_change_of_the_state_is_seen_by_autograd(native_ops, device):
+    """A backward that needs the state as it was before the call is refused."""
+    tensors, state = _inputs(1, 1, 70, 64, 16, "contiguous", device)
+    scale = torch.ones_like(state, requires_grad=True)
+    loss = (state * scale).sum()
+    with torch.no_grad():
+        assert synthetic_model._delta_kernel_takes(*tensors, state, 64)
+        synthetic_model.gated_delta_chunked(*tensors, state)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
+    with torch.inference_mode():
+        inference = state.clone()
+    with pytest.raises(RuntimeError, match="[Ii]nference tensor"):
+        synthetic_model.gated_delta_chunked(*tensors, inference)
+
+
 @pytest.mark.parametrize("b,t,channels,width,ld", [(1, 1, 64, 4, 80), (2, 2, 64, 3, 70), (3, 3, 66, 4, 66),
                                                    (2, 16, 514, 2, 520), (1, 49, 1026, 4, 1030)])
 def test_conv_tokens_equals_the_elementwise_form(native_ops, device, b, t, channels, width, ld):

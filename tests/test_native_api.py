@@ -83,6 +83,19 @@ def test_meta_shapes():
     assert e.shape == (2, 3, 64) and e.dtype == torch.bfloat16
 
 
+def test_prefill_state_updates_count_as_in_place_changes():
+    """As the torch operations they stand in for: the version of the state moves on."""
+    native.load_extension()
+    ops, meta = torch.ops.vllm_ascend_hif8, dict(device="meta")
+    state = torch.empty(1, 2, 64, 16, **meta)
+    k, v, g = torch.empty(1, 2, 5, 64, **meta), torch.empty(1, 2, 5, 16, **meta), torch.empty(1, 2, 5, **meta)
+    assert ops.hif8_gated_delta(k, k, v, g, g, state).shape == v.shape and state._version == 1
+    conv = torch.empty(2, 8, 3, dtype=torch.bfloat16, **meta)
+    out = ops.hif8_conv_tokens(torch.empty(2, 5, 12, dtype=torch.bfloat16, **meta),
+                               torch.empty(8, 4, dtype=torch.bfloat16, **meta), conv)
+    assert out.shape == (2, 5, 8) and conv._version == 1
+
+
 def test_decode_glue_meta_shapes():
     native.load_extension()
     ops = torch.ops.vllm_ascend_hif8
