@@ -26,8 +26,9 @@ codes took two (MI355X, per projection: 24 rows 7.7 -> 4.5 us, 512 rows 10.1
 -> 6.0).
 ``HIF8_STATIC_FUSED_SINGLE_ROW=0`` or ``HIF8_STATIC_FUSED_ROWS=0`` restores
 the reference's routing (static_quant -> soft_linear unless
-``HIF8_STATIC_FUSED_GENERATION=1``, M <= 4, K < 1024, scheme.py:183-190);
-``HIF8_STATIC_FUSED_ROWS=1`` fuses one row only.  The routing changes which
+``HIF8_STATIC_FUSED_GENERATION=1``, M <= 4, K < 1024, scheme.py:183-190) at
+every M; ``HIF8_STATIC_FUSED_ROWS=1`` fuses one row only of the decode-sized
+inputs.  The routing changes which
 kernels run, not the outputs (equal bit for bit).
 
 ``HIF8_PREFILL_BF16_WEIGHTS=1`` (read in ``process_weights_after_loading``)
@@ -75,10 +76,9 @@ def _fused_rows() -> int:
 
 
 def _fuse_prefill_quant() -> bool:
-    """Whether more than four rows on the GPU run static quant and GEMM as one
-    op; any explicit row routing asks for the reference's two stages instead."""
-    return (os.environ.get(_STATIC_FUSED_SINGLE_ROW_ENV, "1") != "0"
-            and not os.environ.get(_STATIC_FUSED_ROWS_ENV))
+    """Whether more than four rows on the GPU run static quant and GEMM as one op:
+    unless either variable restores the reference's two stages."""
+    return _fused_rows() > 0
 
 
 def _static_scale_factor() -> float:

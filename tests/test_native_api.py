@@ -9,7 +9,7 @@ from unittest.mock import patch
 import pytest
 import torch
 
-from hif8_rocm import native
+from hif8_rocm import native, scheme
 from hif8_rocm.scheme import STATIC_QUANT_TYPE, W8A8HiFloat8StaticLinearMethod
 
 
@@ -344,6 +344,19 @@ def test_decode_row_fusion_is_the_default_with_an_opt_out(clean_env):
         if want_fused:
             fused.assert_called_once_with(x, layer.weight, layer.input_scale, layer.weight_scale, None,
                                           output_dtype=x.dtype)
+
+
+@pytest.mark.parametrize("flag,rows_env,fused", [
+    (None, None, True), (None, "", True), (None, "4", True), (None, "1", True), (None, "9", True), ("1", None, True),
+    (None, "0", False), (None, "-1", False), ("0", None, False), ("0", "4", False),
+])
+def test_prefill_quant_fusion_follows_the_reference_routing_switches(clean_env, flag, rows_env, fused):
+    """The row count of the decode fusion leaves the prefill alone; only the values
+    that restore the reference's two stages (0) turn its fused quant off."""
+    for var, val in (("HIF8_STATIC_FUSED_SINGLE_ROW", flag), ("HIF8_STATIC_FUSED_ROWS", rows_env)):
+        if val is not None:
+            os.environ[var] = val
+    assert scheme._fuse_prefill_quant() == fused
 
 
 def test_prefill_bf16_weights_route_only_large_m(clean_env):
