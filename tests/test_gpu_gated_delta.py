@@ -3,9 +3,12 @@ token-by-token definition in float64."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
+from conftest import PKG_ROOT
 from hif8_rocm import synthetic_model
 
 pytestmark = pytest.mark.gpu
@@ -50,6 +53,33 @@ def test_gated_delta_matches_the_recurrence(native_ops, device, b, h, t, dk, dv,
     # FP32 sums of up to 128 products per term, a few terms deep: ~2^-24 sqrt(128) each.
     for x, y in ((got, want), (state, want_state)):
         assert x.dtype == torch.float32 and float((x.double() - y).norm() / y.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("b,kh,rep,t,dk,dv", [(2, 3, 2, 70, 64, 32), (1, 2, 4, 130, 128, 128)])
+def test_gated_delta_of_fewer_key_heads(native_ops, device, b, kh, rep, t, dk, dv):
+    """The C entry with k_heads < heads, q and k [B, T, k_heads, dk] as a layer holds
+    them: value head h reads key head h / rep, bit for bit as if they were repeated."""
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+    lib = ctypes.CDLL(str(PKG_ROOT / "hif8_rocm" / "libhif8_rocm.so"))
+    lib.hif8_last_error.restype = ctypes.c_char_p
+    lib.hif8_gated_delta_workspace_size.argtypes, lib.hif8_gated_delta_workspace_size.restype = [i64] * 5, ctypes.c_size_t
+    lib.hif8_gated_delta.argtypes = [ptr] * 8 + [i64] * 6 + [ptr, ctypes.c_size_t, ptr]
+    h = kh * rep
+    (q, k, _, _, _), _ = _inputs(b, kh, t, dk, dv, "tokens_first", device)
+    (_, _, v, g, beta), state = _inputs(b, h, t, dk, dv, "tokens_first", device)
+    want_state = state.clone()
+    want = torch.ops.vllm_ascend_hif8.hif8_gated_delta(q.repeat_interleave(rep, dim=1), k.repeat_interleave(rep, dim=1),
+                                                       v, g, beta, want_state)
+    out = torch.empty(b, t, h, dv, device=device).transpose(1, 2)
+    strides = (i64 * 18)(*[x.stride(i) for x in (q, k, v, g, beta, out) for i in range(3)])
+    need = lib.hif8_gated_delta_workspace_size(b, h, t, dk, dv)
+    ws = torch.empty(need, dtype=torch.uint8, device=device)
+    torch.cuda.synchronize()
+    pointers = [ptr(x.data_ptr()) for x in (q, k, v, g, beta)]
+    assert lib.hif8_gated_delta(*pointers, strides, ptr(state.data_ptr()), ptr(out.data_ptr()), b, h, kh, t, dk, dv,
+                                ptr(ws.data_ptr()), need, None) == 0, lib.hif8_last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(state, want_state)
 
 
 def test_gated_delta_leaves_autograd_and_other_types_to_torch(native_ops, device):
