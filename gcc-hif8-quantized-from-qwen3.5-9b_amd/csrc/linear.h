@@ -73,8 +73,9 @@ int describe_gemv(int64_t m, int64_t n, int64_t k, int act_kind, char *name, siz
 // the chip split K over several blocks; without one they run unsplit.
 int launch_gemm(const LinearArgs &a);
 size_t gemm_workspace_size(int64_t m, int64_t n, int64_t k);
-// gemm_workspace_size, and for K % 64 != 0 the workspace with which the call
-// runs on the matrix cores (any smaller one: one thread per output).
+// gemm_workspace_size, and at least the bf16 activation fragments with which a
+// call of K % 64 != 0 or of unaligned operands runs on the matrix cores (any
+// smaller one: one thread per output); 0 where the call ends sooner without.
 size_t gemm_scratch_size(int64_t m, int64_t n, int64_t k);
 // The GEMM with the weight already decoded to bf16 (a.weight_bf16; a.weight is
 // not read): the activation codes are decoded into the workspace and both

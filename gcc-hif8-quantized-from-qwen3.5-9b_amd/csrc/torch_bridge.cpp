@@ -192,8 +192,8 @@ at::Tensor SoftHif8Gemv(const at::Tensor &activation, const at::Tensor &weight, 
                         const at::Tensor &channel_scale, const c10::optional<at::Tensor> &bias,
                         at::ScalarType output_dtype) {
   if (activation.dim() == 2 && activation.size(1) % 16 != 0) {
-    // Rows the GEMV cannot stream in 16-byte chunks: the GEMM's few-row kernel,
-    // as soft_hif8_gemm runs them.
+    // Rows the GEMV cannot stream in 16-byte chunks: as soft_hif8_gemm runs them, on
+    // the few-row kernel where that is faster.
     ValidateSoftLinear(activation, weight, token_scale, channel_scale, bias, output_dtype, true);
     return SoftHif8Gemm(activation, weight, token_scale, channel_scale, bias, output_dtype);
   }
@@ -352,7 +352,8 @@ at::Tensor SoftHif8StaticFusedGemm(const at::Tensor &activation, const at::Tenso
   }
   TORCH_CHECK(output_dtype == at::ScalarType::Half || output_dtype == at::ScalarType::BFloat16,
               "output_dtype must be torch.float16 or torch.bfloat16");
-  // Rows the GEMV cannot stream in 16-byte chunks run as more rows do.
+  // Rows the GEMV cannot stream in 16-byte chunks: as more rows do, or (few
+  // products) one output per wavefront after all, as launch_gemm_static picks.
   if (activation.size(1) % 16 != 0)
     return Hif8StaticLinear(activation, weight, fixed_scale, channel_scale, bias, output_dtype);
   const c10::OptionalDeviceGuard guard(device);
