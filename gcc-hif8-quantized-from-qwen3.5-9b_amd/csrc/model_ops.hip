@@ -883,7 +883,7 @@ extern "C" int hif8_qk_norm_rope(const uint16_t *qkv, const uint16_t *q_norm, co
                                  int64_t num_kv_heads, int64_t head_size, int64_t rotary_dim, float eps,
                                  hif8_stream_t stream) {
   clear_error();
-  if (!qkv || !q_norm || !k_norm || !pos || !inv_freq || !q_out || !k_out || !v_out ||
+  if (!qkv || !q_norm || !k_norm || !pos || (!inv_freq && rotary_dim > 0) || !q_out || !k_out || !v_out ||
       (slots && !block_table && max_blocks > 0))
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope: null pointer argument");
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||
@@ -905,7 +905,8 @@ extern "C" int hif8_qk_norm_rope_cache(const uint16_t *qkv, const uint16_t *q_no
                                        int64_t num_kv_heads, int64_t head_size, int64_t rotary_dim, float eps,
                                        hif8_stream_t stream) {
   clear_error();
-  if (!qkv || !q_norm || !k_norm || !pos || !inv_freq || !block_table || !q_out || !key_cache || !value_cache ||
+  if (!qkv || !q_norm || !k_norm || !pos || (!inv_freq && rotary_dim > 0) || !block_table || !q_out || !key_cache ||
+      !value_cache ||
       !key_scale || !value_scale)
     return fail(HIF8_ERR_INVALID_ARGUMENT, "hif8_qk_norm_rope_cache: null pointer argument");
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_size <= 0 || head_size > kHeadThreads ||

@@ -653,3 +653,28 @@ def test_prefill_glue_kernels_match_the_torch_prefill(model, device, monkeypatch
     assert float((caches[0] != want_caches[0]).float().mean()) < 0.01 and torch.equal(caches[1], want_caches[1])
     for p, q in zip(mix, want_mix):
         torch.testing.assert_close(p.float(), q.float(), rtol=2e-2, atol=2e-2)
+
+
+def test_model_without_rotary_dims(native_ops, device):
+    """rotary_dim 0: a prefill and a decode step run, q and k normed and not rotated."""
+    from hif8_rocm.synthetic_model import HybridConfig, HybridModel, rms_norm
+
+    model = HybridModel(HybridConfig(**dict(TINY, layers=1, full_attention_interval=1, rotary_dim=0)), device, seed=4)
+    model.calibrate(batch=1, tokens=16)
+    c, b, t = model.cfg, 2, 6
+    st = model.new_state(b, t + 1)
+    st.seq_lens.fill_(t)
+    ids = torch.randint(0, c.vocab, (b, t), device=device)
+    pos = torch.arange(t, device=device).expand(b, t).contiguous()
+    assert bool(torch.isfinite(model.forward(st, ids, pos, decode=False)).all())
+    st.seq_lens.add_(1)
+    assert bool(torch.isfinite(model.forward(st, ids[:, :1].contiguous(), pos[:, -1:] + 1, decode=True)).all())
+    L = model.layers[0]
+    qkv = torch.randn(3, (c.heads + 2 * c.kv_heads) * c.head_dim, device=device).to(torch.bfloat16)
+    q, k, _, _ = torch.ops.vllm_ascend_hif8.hif8_qk_norm_rope(
+        qkv, L["q_norm"], L["k_norm"], torch.arange(3, device=device), model.inv_freq, st.block_table[:1].repeat(3, 1),
+        c.block_size, c.heads, c.kv_heads, c.head_dim, c.rms_eps)
+    heads = qkv.reshape(3, -1, c.head_dim)[:, :c.heads + c.kv_heads]
+    # Sums in another order: one bf16 rounding step apart at most.
+    torch.testing.assert_close(torch.cat([q, k], dim=1).float(), rms_norm(heads, L["q_norm"], c.rms_eps).float(),
+                               rtol=2 ** -7, atol=1e-6)
